@@ -4,11 +4,14 @@
 // steady state (rho, u, v, T): Linear(5,W) + SiLU, (L-1) x [Linear(W,W) +
 // SiLU], Linear(W,4).  Weights and activations are BF16, accumulation and
 // master weights FP32, optimiser Adam.  The W x W layers (all but ~1% of the
-// work) run on gfx950's v_mfma_f32_32x32x16_bf16 through one tiled GEMM kernel with
-// three epilogues: forward (bias + SiLU, keeps the pre-activation), backward
-// data (times SiLU' of the previous pre-activation) and backward weight
-// (split-K partials over the batch).  The 5-wide input and 4-wide output
-// layers are plain FP32 SIMT kernels.  The network only seeds the solver's
+// work) run on gfx950's v_mfma_f32_32x32x16_bf16.  Up to width kMaxFused the
+// fused kernels of mlp_net.hpp carry 32 rows per wavefront through the whole
+// network in registers.  Wider networks, whose activations do not fit a
+// wavefront's registers, run layer by layer through one tiled GEMM kernel
+// with three epilogues: forward (bias + SiLU, keeps the pre-activation),
+// backward data (times SiLU' of the previous pre-activation) and backward
+// weight (split-K partials over the batch), the 5-wide input and 4-wide
+// output layers through plain FP32 SIMT kernels.  The network only seeds the solver's
 // initial Maxwellian (dgbgk_seed_maxwellian); it has no counterpart in the
 // reference.
 #include <hip/hip_runtime.h>
@@ -365,10 +368,37 @@ __global__ void __launch_bounds__(256) k_wgrad_in(const bf16* __restrict__ dZ, i
   }
 }
 
-// Adam on FP32 master parameters, then the BF16 copy the kernels read
+}  // namespace mlp
+}  // namespace dgbgk
+
+#include "mlp_net.hpp"
+
+namespace dgbgk {
+namespace mlp {
+
+// the BF16 parameters the kernels read: packed as the master copy, and for
+// the fused kernels the hidden weights again as forward and backward
+// operands (pack_index)
+struct Bf16Params {
+  bf16 *pb, *wf, *wb;  // wf, wb null without the fused kernels
+  size_t base, per;    // parameters of the input layer, of a hidden layer
+  int width, hidden;
+};
+__device__ __forceinline__ void put_bf16(const Bf16Params& q, size_t i, float x) {
+  const bf16 h = f2bf(x);
+  q.pb[i] = h;
+  if (!q.wf || i < q.base) return;
+  const size_t j = i - q.base, l = j / q.per, r = j % q.per, ww = (size_t)q.width * q.width;
+  if (l + 1 >= (size_t)q.hidden || r >= ww) return;
+  const int o = (int)(r / q.width), k = (int)(r % q.width);
+  q.wf[l * ww + pack_index(o, k, q.width)] = h;
+  q.wb[l * ww + pack_index(k, o, q.width)] = h;
+}
+
+// Adam on FP32 master parameters, then the BF16 copies the kernels read
 __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
                        const float* __restrict__ g, size_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2, bf16* __restrict__ pb) {
+                       float eps, float c1, float c2, Bf16Params q) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -378,25 +408,21 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __re
   v[i] = vi;
   const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   p[i] = pi;
-  pb[i] = f2bf(pi);
+  put_bf16(q, i, pi);
 }
 
-__global__ void k_to_bf16(const float* __restrict__ p, size_t n, bf16* __restrict__ pb) {
+__global__ void k_to_bf16(const float* __restrict__ p, size_t n, Bf16Params q) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) pb[i] = f2bf(p[i]);
+  if (i < n) put_bf16(q, i, p[i]);
 }
 
-// batch gather with a counter-based hash of (seed, step, row)
+// batch gather of the rows drawn_row names
 __global__ void k_gather(const float* __restrict__ X, const float* __restrict__ Y, long ns,
                          int fin, int fout, int rows, unsigned seed, unsigned step,
                          float* __restrict__ Xb, float* __restrict__ Yb) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= rows) return;
-  unsigned long long h = ((unsigned long long)seed << 32) ^ ((unsigned long long)step << 20) ^
-                         (unsigned long long)r;
-  h ^= h >> 33; h *= 0xff51afd7ed558ccdULL; h ^= h >> 33; h *= 0xc4ceb9fe1a85ec53ULL;
-  h ^= h >> 33;
-  const long idx = (long)(h % (unsigned long long)ns);
+  const long idx = drawn_row(seed, step, r, ns);
   for (int k = 0; k < fin; ++k) Xb[(size_t)r * fin + k] = X[(size_t)idx * fin + k];
   for (int k = 0; k < fout; ++k) Yb[(size_t)r * fout + k] = Y[(size_t)idx * fout + k];
 }
@@ -443,6 +469,12 @@ struct dgbgk_mlp {
   hipStream_t stream = nullptr;
   float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // master, Adam, gradient
   bf16* pb = nullptr;                                             // BF16 parameters
+  // fused kernels (width <= kMaxFused): hidden weights as operands, the
+  // kernels' activations, pre-activations and dZ, partial sums
+  bool fused = false;
+  bf16 *wf = nullptr, *wb = nullptr;
+  uintx4 *nZ = nullptr, *nA = nullptr, *nD = nullptr;
+  float *pw = nullptr, *pin = nullptr, *pout = nullptr, *pbias = nullptr;
   std::vector<bf16*> Z, A;         // per hidden layer, [batch][width]
   bf16 *dZa = nullptr, *dZb = nullptr;
   float *Xb = nullptr, *Yb = nullptr, *Yout = nullptr, *dY = nullptr;
@@ -468,6 +500,79 @@ int wsplits(int rows) {
   int s = std::min(64, std::max(1, rows / 1024));
   while (s > 1 && rows % (s * kKC) != 0) --s;
   return s;
+}
+
+Bf16Params bf16_params(const dgbgk_mlp* h) {
+  return Bf16Params{h->pb, h->wf, h->wb, h->woff[1], h->woff[2] - h->woff[1], h->width,
+                    h->hidden};
+}
+
+// Wavefronts per block of k_net: four share the streamed weights once there
+// are two such blocks for each of the 256 CUs (65,536 rows), two below
+// 32,768 rows, where the chip is not filled and shorter blocks spread.
+int net_waves(int rows) { return rows >= 32768 ? 4 : 2; }
+int net_blocks(int rows) {
+  const int per = 32 * net_waves(rows);
+  return (rows + per - 1) / per;
+}
+
+template <int W, bool kTrain>
+void launch_net_w(dgbgk_mlp* h, const NetArgs& a) {
+  const dim3 g(net_blocks(a.rows)), b(64 * net_waves(a.rows));
+  // the shipped networks' 5 inputs and 4 outputs, or any up to 8
+  const bool five = a.fin <= 5 && a.fout <= 4;
+  if (b.x == 256) {
+    if (five) hipLaunchKernelGGL((k_net<W, 4, kTrain, 5, 4>), g, b, 0, h->stream, a);
+    else hipLaunchKernelGGL((k_net<W, 4, kTrain, 8, 8>), g, b, 0, h->stream, a);
+  } else {
+    if (five) hipLaunchKernelGGL((k_net<W, 2, kTrain, 5, 4>), g, b, 0, h->stream, a);
+    else hipLaunchKernelGGL((k_net<W, 2, kTrain, 8, 8>), g, b, 0, h->stream, a);
+  }
+}
+template <bool kTrain>
+int launch_net(dgbgk_mlp* h, const NetArgs& a) {
+  switch (h->width) {
+    case 64: launch_net_w<64, kTrain>(h, a); break;
+    case 128: launch_net_w<128, kTrain>(h, a); break;
+    case 192: launch_net_w<192, kTrain>(h, a); break;
+    default: launch_net_w<256, kTrain>(h, a); break;
+  }
+  MCK(hipGetLastError());
+  return 0;
+}
+
+NetArgs net_args(dgbgk_mlp* h, int rows) {
+  NetArgs a{};
+  a.rows = rows;
+  a.fin = h->fin; a.fout = h->fout; a.hidden = h->hidden;
+  a.pb = h->pb; a.p = h->p; a.wf = h->wf; a.wb = h->wb;
+  a.Y = h->Yout; a.loss_part = h->loss_part;
+  a.Z = h->nZ; a.A = h->nA; a.D = h->nD;
+  a.act4 = (size_t)h->batch * h->width / 8;
+  a.pin = h->pin; a.pout = h->pout; a.pbias = h->pbias;
+  return a;
+}
+
+// loss partials (net_blocks of them) and the gradient of the mean squared
+// error into h->g
+int net_loss_grad(dgbgk_mlp* h, const NetArgs& a) {
+  int st = launch_net<true>(h, a);
+  if (st) return st;
+  const int W = h->width, L1 = h->hidden - 1, sp = wsplits(a.rows), rper = a.rows / sp;
+  const dim3 g(sp, L1), b(256);
+  switch (W) {
+    case 64: hipLaunchKernelGGL(k_wgrad<64>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
+    case 128: hipLaunchKernelGGL(k_wgrad<128>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
+    case 192: hipLaunchKernelGGL(k_wgrad<192>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
+    default: hipLaunchKernelGGL(k_wgrad<256>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
+  }
+  NetReduce r{h->pw, h->pbias, h->pin, h->pout, h->g, W, h->hidden, h->fin, h->fout, sp,
+              net_blocks(a.rows)};
+  const int nb = L1 * (W * W + W) / kRedCols + W * (h->fin + 1) / kRedCols +
+                 (h->fout * (W + 1) + kRedCols - 1) / kRedCols;
+  hipLaunchKernelGGL(k_reduce_net, dim3(nb), b, 0, h->stream, r);
+  MCK(hipGetLastError());
+  return 0;
 }
 
 int forward(dgbgk_mlp* h, int rows, bool with_loss) {
@@ -546,7 +651,7 @@ int adam(dgbgk_mlp* h, float lr) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - std::pow(b1, (float)h->step), c2 = 1.0f - std::pow(b2, (float)h->step);
   hipLaunchKernelGGL(k_adam, dim3((unsigned)((h->nparams + 255) / 256)), dim3(256), 0, h->stream,
-                     h->p, h->m, h->v, h->g, h->nparams, lr, b1, b2, eps, c1, c2, h->pb);
+                     h->p, h->m, h->v, h->g, h->nparams, lr, b1, b2, eps, c1, c2, bf16_params(h));
   MCK(hipGetLastError());
   return 0;
 }
@@ -602,22 +707,39 @@ int dgbgk_mlp_create(int fin, int width, int hidden, int fout, int batch, dgbgk_
   st |= dalloc(h, &h->v, h->nparams);
   st |= dalloc(h, &h->g, h->nparams);
   st |= dalloc(h, &h->pb, h->nparams);
-  h->Z.assign(hidden, nullptr);
-  h->A.assign(hidden, nullptr);
-  for (int l = 0; l < hidden; ++l) {
-    st |= dalloc(h, &h->Z[l], act);
-    st |= dalloc(h, &h->A[l], act);
-  }
-  st |= dalloc(h, &h->dZa, act);
-  st |= dalloc(h, &h->dZb, act);
+  h->fused = width <= kMaxFused;
   st |= dalloc(h, &h->Xb, (size_t)batch * fin);
   st |= dalloc(h, &h->Yb, (size_t)batch * fout);
   st |= dalloc(h, &h->Yout, (size_t)batch * fout);
-  st |= dalloc(h, &h->dY, (size_t)batch * fout);
-  const int nch = (batch + kRowChunk - 1) / kRowChunk;
-  h->part_n = std::max({(size_t)64 * width * width, (size_t)nch * width * (fin + 1),
-                        (size_t)nch * fout * (width + 1), (size_t)nch * width});
-  st |= dalloc(h, &h->part, h->part_n);
+  if (h->fused) {
+    const size_t L1 = hidden - 1, ww = (size_t)width * width, act4 = act / 8;
+    // the most blocks and splits any row count up to batch launches
+    const size_t nblk = std::max(net_blocks(batch), net_blocks(std::min(batch, 32768 - kTile)));
+    const size_t sp = std::max(1, std::min(64, batch / 1024));
+    st |= dalloc(h, &h->wf, L1 * ww);
+    st |= dalloc(h, &h->wb, L1 * ww);
+    st |= dalloc(h, &h->nZ, hidden * act4);
+    st |= dalloc(h, &h->nA, L1 * act4);
+    st |= dalloc(h, &h->nD, L1 * act4);
+    st |= dalloc(h, &h->pw, L1 * sp * ww);
+    st |= dalloc(h, &h->pin, nblk * width * (fin + 1));
+    st |= dalloc(h, &h->pout, nblk * fout * (width + 1));
+    st |= dalloc(h, &h->pbias, L1 * nblk * width);
+  } else {
+    h->Z.assign(hidden, nullptr);
+    h->A.assign(hidden, nullptr);
+    for (int l = 0; l < hidden; ++l) {
+      st |= dalloc(h, &h->Z[l], act);
+      st |= dalloc(h, &h->A[l], act);
+    }
+    st |= dalloc(h, &h->dZa, act);
+    st |= dalloc(h, &h->dZb, act);
+    st |= dalloc(h, &h->dY, (size_t)batch * fout);
+    const int nch = (batch + kRowChunk - 1) / kRowChunk;
+    h->part_n = std::max({(size_t)64 * width * width, (size_t)nch * width * (fin + 1),
+                          (size_t)nch * fout * (width + 1), (size_t)nch * width});
+    st |= dalloc(h, &h->part, h->part_n);
+  }
   st |= dalloc(h, &h->loss_part, (size_t)(batch + 63) / 64);
   st |= dalloc(h, &h->losses, 1);
   if (st) return bail(st);
@@ -647,7 +769,7 @@ int dgbgk_mlp_set_params(dgbgk_mlp* h, const float* params) {
   if (!h || !params) return mfail(DGBGK_ERR_ARG, "null argument");
   MCK(hipMemcpyAsync(h->p, params, h->nparams * sizeof(float), hipMemcpyHostToDevice, h->stream));
   hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((h->nparams + 255) / 256)), dim3(256), 0,
-                     h->stream, h->p, h->nparams, h->pb);
+                     h->stream, h->p, h->nparams, bf16_params(h));
   MCK(hipMemsetAsync(h->m, 0, h->nparams * sizeof(float), h->stream));
   MCK(hipMemsetAsync(h->v, 0, h->nparams * sizeof(float), h->stream));
   h->step = 0;
@@ -668,10 +790,19 @@ int dgbgk_mlp_forward(dgbgk_mlp* h, long n, const float* x, float* y) {
   for (long r0 = 0; r0 < n; r0 += h->batch) {
     const int rows = (int)std::min<long>(h->batch, n - r0);
     const int padded = (rows + kTile - 1) / kTile * kTile;
-    MCK(hipMemsetAsync(h->Xb, 0, (size_t)padded * h->fin * sizeof(float), h->stream));
+    if (!h->fused)
+      MCK(hipMemsetAsync(h->Xb, 0, (size_t)padded * h->fin * sizeof(float), h->stream));
     MCK(hipMemcpyAsync(h->Xb, x + (size_t)r0 * h->fin, (size_t)rows * h->fin * sizeof(float),
                        hipMemcpyHostToDevice, h->stream));
-    int st = forward(h, padded, false);
+    int st = 0;
+    if (h->fused) {
+      NetArgs a = net_args(h, padded);
+      a.X = h->Xb;
+      a.n = rows;
+      st = launch_net<false>(h, a);
+    } else {
+      st = forward(h, padded, false);
+    }
     if (st) return st;
     MCK(hipMemcpyAsync(y + (size_t)r0 * h->fout, h->Yout, (size_t)rows * h->fout * sizeof(float),
                        hipMemcpyDeviceToHost, h->stream));
@@ -691,10 +822,20 @@ int dgbgk_mlp_loss_grad(dgbgk_mlp* h, int rows, const float* x, const float* y, 
                      h->stream));
   MCK(hipMemcpyAsync(h->Yb, y, (size_t)rows * h->fout * sizeof(float), hipMemcpyHostToDevice,
                      h->stream));
-  if ((st = forward(h, rows, true))) return st;
-  if ((st = backward(h, rows))) return st;
-  hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, h->stream, h->loss_part,
-                     (rows + 63) / 64, h->losses);
+  int nloss = (rows + 63) / 64;
+  if (h->fused) {
+    NetArgs a = net_args(h, rows);
+    a.X = h->Xb;
+    a.T = h->Yb;
+    a.n = rows;
+    if ((st = net_loss_grad(h, a))) return st;
+    nloss = net_blocks(rows);
+  } else {
+    if ((st = forward(h, rows, true))) return st;
+    if ((st = backward(h, rows))) return st;
+  }
+  hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, h->stream, h->loss_part, nloss,
+                     h->losses);
   if (loss)
     MCK(hipMemcpyAsync(loss, h->losses, sizeof(float), hipMemcpyDeviceToHost, h->stream));
   if (grad)
@@ -735,15 +876,27 @@ int dgbgk_mlp_train(dgbgk_mlp* h, int steps, float lr, unsigned seed, float* los
     MCK(hipMalloc((void**)&dl, std::max(steps, 1) * sizeof(float)));
   }
   int st = 0;
+  const int nloss = h->fused ? net_blocks(rows) : (rows + 63) / 64;
   for (int s = 0; s < steps && !st; ++s) {
-    hipLaunchKernelGGL(k_gather, dim3((rows + 255) / 256), dim3(256), 0, h->stream, h->Xall,
-                       h->Yall, h->nall, h->fin, h->fout, rows, seed, (unsigned)(h->step + 1),
-                       h->Xb, h->Yb);
-    st = forward(h, rows, true);
-    if (!st) st = backward(h, rows);
+    if (h->fused) {
+      NetArgs a = net_args(h, rows);
+      a.X = h->Xall;
+      a.T = h->Yall;
+      a.n = h->nall;
+      a.gather = 1;
+      a.seed = seed;
+      a.step = (unsigned)(h->step + 1);
+      st = net_loss_grad(h, a);
+    } else {
+      hipLaunchKernelGGL(k_gather, dim3((rows + 255) / 256), dim3(256), 0, h->stream, h->Xall,
+                         h->Yall, h->nall, h->fin, h->fout, rows, seed, (unsigned)(h->step + 1),
+                         h->Xb, h->Yb);
+      st = forward(h, rows, true);
+      if (!st) st = backward(h, rows);
+    }
     if (!st && dl)
-      hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, h->stream, h->loss_part,
-                         (rows + 63) / 64, dl + s);
+      hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, h->stream, h->loss_part, nloss,
+                         dl + s);
     if (!st) st = adam(h, lr);
   }
   if (!st && dl) {
