@@ -94,6 +94,24 @@ __device__ __forceinline__ T node_increment(bool cmminc, T mdt, T rhs, T cold, R
   return d;
 }
 
+// max(m, |a|, |b|, |c|), NaNs skipped as fmax does.  Written with the
+// instruction's |.| operands: fmax of a fabs compiles to an and, a
+// canonicalising max and the max (9 of the update's 36 FP32 epilogue
+// instructions per element and ordinate).
+__device__ __forceinline__ float absmax(float m, float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(m) : "v"(r), "v"(c));
+  return m;
+}
+__device__ __forceinline__ double absmax(double m, double a, double b, double c) {
+  double r;
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(a));
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(m) : "v"(r), "v"(b));
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(c));
+  return r;
+}
+
 __device__ __forceinline__ float dexp(float x) { return __expf(x); }
 __device__ __forceinline__ double dexp(double x) { return exp(x); }
 
@@ -207,8 +225,11 @@ template <typename T>
 struct SlotState {
   T gx[3], gy[3], pA[3], pB[3], pU[3], pV[3], pMd[3];  // phase A (all slots)
   T gxa[3], gya[3], mdt, nx[3], ny[3];                 // phase B (owned slots)
-  int info[3], mask, wsl, e;
-  int nb1[3], nb2[3];  // LDS index (4 slot + node) of the neighbour's values at k, k1
+  int mask, wsl, e;
+  // LDS index (4 slot + node) of the neighbour's values at k, k1; a boundary
+  // side reads its own element's, an FP32 inflow side the slot of zeros
+  int nb1[3], nb2[3];
+  bool inflow[3];      // FP32: the own values are never upwind (a lane mask, in SGPRs)
   float dph;           // FP32 store dither: the element's fixed phase
   bool owned, active;
 };
@@ -226,45 +247,102 @@ __device__ __forceinline__ void store4<double>(double* p, double a, double b, do
   reinterpret_cast<double2*>(p)[1] = make_double2(c, d);
 }
 
-// One ordinate v of one slot.  f: the slot's three node values at v; sf:
-// this ordinate's LDS buffer, [slot][4] = g = f - U at the three nodes and
-// a zero.  ph: the ordinate's and step's dither phase, dsc0/dsc1 the
-// dither's scale (zero without it).
-// Contains the block's one barrier per ordinate, so every thread of the
-// block calls it for every v.
-template <typename T, bool kMom, bool kCM>
-__device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotState<T>& s,
-                                                int v, T ux, T uy, T fin, float ph,
-                                                float dsc0, float dsc1,
-                                                const T (&f)[3],
-                                                T* __restrict__ sf, T dte, T& res, T& chg,
-                                                double wv, double wcx, double wcy,
-                                                double (&m0)[3], double (&m1)[3],
-                                                double (&m2)[3]) {
+// The scalars of one ordinate: a row of vrow, read by scalar loads one
+// ordinate ahead, right after the barrier: a scalar load still in flight at
+// the barrier would be waited for there (one counter for scalar and LDS
+// operations), before every wavefront's second half.  With the row, the
+// upwind select on one compare (no side has a case of its own) and absmax,
+// an element and ordinate takes 116 vector and 39 scalar instructions in
+// FP32 (154 and 77 before) and 137 vector ones in FP64 (172).  FP32 is bound
+// by them: update 325 -> 306 us at 101,753 x 512, 351 -> 326 us at 25,781 x
+// 2048; FP64 by memory: 626 -> 629 us.
+template <typename T>
+struct OrdRow {
+  T ux, uy, fin, ph;   // velocity, inflow value, FP32 store dither phase
+  double w, wcx, wcy;  // moment weights
+};
+template <typename T, bool kMom>
+__device__ __forceinline__ OrdRow<T> ord_row(const T* vrow, int v) {
+  const T* r = vrow + (size_t)v * (kOrdRow / sizeof(T));
+  OrdRow<T> o;
+  o.ux = ldc(r, 0);
+  o.uy = ldc(r, 1);
+  o.fin = ldc(r, 2);
+  o.ph = sizeof(T) == 4 ? ldc(r, 3) : T(0);
+  const double* d = reinterpret_cast<const double*>(r + 4);
+  o.w = kMom ? ldc(d, 0) : 0.0;
+  o.wcx = kMom ? ldc(d, 1) : 0.0;
+  o.wcy = kMom ? ldc(d, 2) : 0.0;
+  return o;
+}
+
+// What the first half of an ordinate leaves for the second.
+template <typename T>
+struct Half {
+  T cold[3], h[3], U;
+  T d1, d2;  // FP32: differences from f_0
+};
+
+// First half of one ordinate of one slot, up to the LDS write.  f: the
+// slot's three node values; sf: this ordinate's LDS buffer, [slot][4] =
+// g = f - U at the three nodes and a zero (FP32: f and U).
+template <typename T>
+__device__ __forceinline__ Half<T> update_first(const SlotState<T>& s, T ux, T uy,
+                                                const T (&f)[3], T* __restrict__ sf, T dte) {
   const int slot = threadIdx.x;
   const T c13 = T(1) / T(3);
+  Half<T> o;
   // collision term times DTE: pMd = MU * DTE (src/getinc.f90:34-41)
   // phase A runs on every slot without a branch: slots without an element
   // hold zero parameters and element 0's f, and nobody reads their result
-  T cold[3], h[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const T dx = s.pU[k] - ux, dy = s.pV[k] - uy;
     const T feq = s.pA[k] * mexp(-s.pB[k] * (dx * dx + dy * dy));
-    cold[k] = s.pMd[k] * (feq - f[k]);
+    o.cold[k] = s.pMd[k] * (feq - f[k]);
   }
-  const T cs = cold[0] + cold[1] + cold[2];
-  T rhs[3], U;
+  const T cs = o.cold[0] + o.cold[1] + o.cold[2];
   if constexpr (sizeof(T) == 8) {
     // GETELC's predictor: U = DTE/2 (div(c f) - (1/3) sum MU (f_eq - f))
     const T sx = s.gx[0] * f[0] + s.gx[1] * f[1] + s.gx[2] * f[2];
     const T sy = s.gy[0] * f[0] + s.gy[1] * f[1] + s.gy[2] * f[2];
-    U = T(0.5) * ((ux * sx + uy * sy) * dte - c13 * cs);
+    o.U = T(0.5) * ((ux * sx + uy * sy) * dte - c13 * cs);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) h[k] = f[k] - U;
-    store4(sf + 4 * slot, h[0], h[1], h[2], T(0));
-    __syncthreads();
-    if (!s.owned) return;
+    for (int k = 0; k < 3; ++k) o.h[k] = f[k] - o.U;
+    store4(sf + 4 * slot, o.h[0], o.h[1], o.h[2], T(0));
+  } else {
+    // FP32: the same operator in exact arithmetic, evaluated on differences
+    // of nearby values so that FP32 rounds the small terms, not f.
+    // Predictor: the gradients sum to zero, so div(c f) takes f - f_0.
+    o.d1 = f[1] - f[0];
+    o.d2 = f[2] - f[0];
+    const T sx = s.gx[1] * o.d1 + s.gx[2] * o.d2;
+    const T sy = s.gy[1] * o.d1 + s.gy[2] * o.d2;
+    o.U = T(0.5) * ((ux * sx + uy * sy) * dte - c13 * cs);
+    // neighbours read raw f and U: each reader forms differences from its
+    // own values before anything is rounded at the size of f
+    store4(sf + 4 * slot, f[0], f[1], f[2], o.U);
+  }
+  return o;
+}
+
+// Second half, after the block's barrier, of the owned slots: ordinate v's
+// fluxes, increment and store.  ph: the ordinate's and step's dither phase,
+// dsc0/dsc1 the dither's scale (zero without it); anyin: the wavefront
+// holds inflow nodes.
+template <typename T, bool kMom, bool kCM>
+__device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotState<T>& s,
+                                              Half<T>& o, int v, const OrdRow<T>& r, float ph,
+                                              float dsc0, float dsc1, bool anyin,
+                                              const T (&f)[3], const T* __restrict__ sf, T& res,
+                                              T& chg, double (&m0)[3], double (&m1)[3],
+                                              double (&m2)[3]) {
+  const T c13 = T(1) / T(3);
+  const T ux = r.ux, uy = r.uy, fin = r.fin, U = o.U;
+  T(&cold)[3] = o.cold;
+  T(&h)[3] = o.h;
+  T rhs[3];
+  if constexpr (sizeof(T) == 8) {
     // volume term (src/getelc.f90:87-117): area * grad N_a . c (mean of f - U)
     const T sm = c13 * (h[0] + h[1] + h[2]);
     const T fx = ux * sm, fy = uy * sm;
@@ -276,16 +354,16 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
     // M2 = [[2,1],[1,2]] and g = f - U of the upwind element.  The reference
     // orients each side once (left element) and subtracts the left element's
     // flux from the right element; with the right element's outward normal
-    // that is the same expression.  Upwind: own values when c.n > 0 (on a
-    // tie the right element's values, as in the reference), always on a
-    // boundary side; inflow and wall sides carry a zero (len/6) n here.
+    // that is the same expression.  Upwind: own values when c.n > 0; on a
+    // tie the flux is zero whichever element's values it takes; on an outflow
+    // side the neighbour's are the own; inflow and wall sides carry a zero
+    // (len/6) n here.
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int k1 = (k + 1) % 3;
-      const int in = s.info[k];
       // w = -(len/6) c.n from the edge's (len/6) n: c.n > 0 exactly when w < 0
       const T w = -(ux * s.nx[k] + uy * s.ny[k]);
-      const bool own = (in & kUpdOwn) || w < T(0) || ((in & kUpdRight) && w == T(0));
+      const bool own = w < T(0);
       // the neighbour's values are read whichever side is upwind (fixed LDS
       // indices, no address arithmetic); the element's own are in registers
       const T n1 = sf[s.nb1[k]], n2 = sf[s.nb2[k]];
@@ -294,35 +372,21 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
       rhs[k1] += w * (g1 + T(2) * g2);
     }
   } else {
-    // FP32: the same operator in exact arithmetic, evaluated on differences
-    // of nearby values so that FP32 rounds the small terms, not f.
-    // Predictor: the gradients sum to zero, so div(c f) takes f - f_0.
-    const T d1 = f[1] - f[0], d2 = f[2] - f[0];
-    const T sx = s.gx[1] * d1 + s.gx[2] * d2;
-    const T sy = s.gy[1] * d1 + s.gy[2] * d2;
-    U = T(0.5) * ((ux * sx + uy * sy) * dte - c13 * cs);
-    // neighbours read raw f and U: each reader forms differences from its
-    // own values before anything is rounded at the size of f
-    store4(sf + 4 * slot, f[0], f[1], f[2], U);
-    __syncthreads();
-    if (!s.owned) return;
     // area grad N_k is half the sum of len n over the element's edges at
     // node k, so the volume term folds into the edges: each edge acts on
     // (upwind g - the element's mean gbar of f - U), the mean about f_0 as
     // gbar = f_0 + db - U with db the mean of (0, d1, d2)
-    const T db = c13 * (d1 + d2);
+    const T db = c13 * (o.d1 + o.d2);
     h[0] = -db;
-    h[1] = d1 - db;
-    h[2] = d2 - db;
-    const T gbar = (f[0] + db) - U;  // an inflow side's upwind values are 0
+    h[1] = o.d1 - db;
+    h[2] = o.d2 - db;
 #pragma unroll
     for (int k = 0; k < 3; ++k) rhs[k] = T(0);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int k1 = (k + 1) % 3;
-      const int in = s.info[k];
       const T w = -(ux * s.nx[k] + uy * s.ny[k]);
-      const bool own = (in & kUpdOwn) || w < T(0) || ((in & kUpdRight) && w == T(0));
+      const bool own = w < T(0) && !s.inflow[k];
       const T n1 = sf[s.nb1[k]], n2 = sf[s.nb2[k]], un = sf[s.nb1[k] | 3];
       const T du = un - U;
       T e1 = ((n1 - f[0]) - db) - du, e2 = ((n2 - f[0]) - db) - du;
@@ -330,9 +394,7 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
       // for all slots), so the upwind choice below is a select, not a
       // divergent branch around the reads per edge
       asm volatile("" : "+v"(e1), "+v"(e2));
-      const bool inflow = (in & kUpdInflow) != 0;
-      const T g1 = own ? (inflow ? -gbar : h[k]) : e1;
-      const T g2 = own ? (inflow ? -gbar : h[k1]) : e2;
+      const T g1 = own ? h[k] : e1, g2 = own ? h[k1] : e2;
       rhs[k] += w * (T(2) * g1 + g2);
       rhs[k1] += w * (g1 + T(2) * g2);
     }
@@ -357,7 +419,9 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
   if constexpr (sizeof(T) == 4) t = fmaf(__builtin_amdgcn_fractf(s.dph + ph), dsc0, dsc1);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    d[k] = node_increment(kCM, s.mdt, rhs[k], cold[k], res);
+    T term = T(0);
+    d[k] = node_increment(kCM, s.mdt, rhs[k], cold[k], term);
+    if (kCM) res = fmax(res, term);
     T dk = d[k];
     if constexpr (sizeof(T) == 4)
       dk = fmaf(t, __uint_as_float(__float_as_uint(f[k]) & 0x7f800000u), dk);
@@ -366,7 +430,8 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
     fn[k] = neg ? T(0) : fn[k];  // NaN stays NaN, as in the reference
     if constexpr (sizeof(T) == 4) cg[k] = neg ? f[k] : T(fabs(d[k]));
   }
-  if (__ballot(s.mask != 0)) {  // inflow nodes: rare; a wave-uniform branch
+  if (!kCM) res = absmax(res, d[0], d[1], d[2]);
+  if (anyin) {  // inflow nodes: rare; a wave-uniform branch
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       if ((s.mask >> k) & 1) {
@@ -376,9 +441,9 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
   }
   if constexpr (sizeof(T) == 8) {  // FP64: the change as stored
 #pragma unroll
-    for (int k = 0; k < 3; ++k) cg[k] = fabs(fn[k] - f[k]);
+    for (int k = 0; k < 3; ++k) cg[k] = fn[k] - f[k];
   }
-  chg = fmax(chg, fmax(fmax(cg[0], cg[1]), cg[2]));
+  chg = absmax(chg, cg[0], cg[1], cg[2]);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     fstore_nt(fo + k, fn[k]);
@@ -387,9 +452,9 @@ __device__ __forceinline__ void update_ordinate(const UpdArgs<T>& a, const SlotS
       // ordinates, in FP64 (wcx = w cx, wcy = w cy; k_moments sums the same
       // products in the same order)
       const double fd = (double)fn[k];
-      m0[k] = fma(wv, fd, m0[k]);
-      m1[k] = fma(wcx, fd, m1[k]);
-      m2[k] = fma(wcy, fd, m2[k]);
+      m0[k] = fma(r.w, fd, m0[k]);
+      m1[k] = fma(r.wcx, fd, m1[k]);
+      m2[k] = fma(r.wcy, fd, m2[k]);
     }
   }
 }
@@ -416,7 +481,13 @@ k_update(UpdArgs<T> a) {
   constexpr int kQ = kDepth + 1;
   // one LDS buffer per queue position: ordinate v + kQ reuses v's buffer
   // after kQ - 1 >= 1 barriers, and the buffer is a compile-time offset
-  __shared__ __align__(16) T s_f[kQ][kS * 4];
+  // (FP32: and a slot of zeros past the threads', the upwind values of an
+  // inflow side: with f = U = 0 there the neighbour's expression is exactly
+  // minus the own element's mean, so no side needs a case of its own)
+  constexpr int kRow = (kS + (sizeof(T) == 4 ? 1 : 0)) * 4;
+  __shared__ __align__(16) T s_f[kQ][kRow];
+  if (sizeof(T) == 4 && threadIdx.x < 4 * kQ)  // read after the first barrier
+    s_f[threadIdx.x / 4][kS * 4 + threadIdx.x % 4] = T(0);
   __shared__ double s_red[8];
   const int logical = xcd_logical(blockIdx.x, gridDim.x);
   const int tile = logical % a.ntiles;
@@ -438,7 +509,7 @@ k_update(UpdArgs<T> a) {
   for (int k = 0; k < 3; ++k) {
     s.gx[k] = s.gy[k] = s.pA[k] = s.pB[k] = s.pU[k] = s.pV[k] = s.pMd[k] = T(0);
     s.gxa[k] = s.gya[k] = s.nx[k] = s.ny[k] = T(0);
-    s.info[k] = kUpdOwn;
+    s.inflow[k] = false;
     s.nb1[k] = 4 * slot + k;
     s.nb2[k] = 4 * slot + (k + 1) % 3;
 
@@ -467,11 +538,14 @@ k_update(UpdArgs<T> a) {
     for (int k = 0; k < 3; ++k) {
       s.gxa[k] = s.gx[k] * area;
       s.gya[k] = s.gy[k] * area;
-      s.info[k] = a.uinfo[k * E + e];
-      if (!(s.info[k] & kUpdOwn)) {  // interior side: the neighbour's slot and nodes
-        const int nbs = s.info[k] >> kUpdSlot;
-        s.nb1[k] = 4 * nbs + ((s.info[k] >> kUpdNbK) & 3);
-        s.nb2[k] = 4 * nbs + ((s.info[k] >> kUpdNbK1) & 3);
+      const int in = a.uinfo[k * E + e];
+      if (!(in & kUpdOwn)) {  // interior side: the neighbour's slot and nodes
+        const int nbs = in >> kUpdSlot;
+        s.nb1[k] = 4 * nbs + ((in >> kUpdNbK) & 3);
+        s.nb2[k] = 4 * nbs + ((in >> kUpdNbK1) & 3);
+      } else if (sizeof(T) == 4 && (in & kUpdInflow)) {
+        s.nb1[k] = s.nb2[k] = 4 * kS;
+        s.inflow[k] = true;
       }
       s.nx[k] = a.unx[k * E + e];
       s.ny[k] = a.uny[k * E + e];
@@ -482,37 +556,24 @@ k_update(UpdArgs<T> a) {
   }
   T res = 0, chg = 0;
 
-  // prime the queue: f and the ordinate's velocity and inflow value for
-  // v0 .. v0+kDepth-1
-  T q[kQ][3], qx[kQ], qy[kQ], qi[kQ];
-  float qp[kQ];  // FP32 store dither: the ordinate's phase plus this step's
-  double qw[kQ], qcx[kQ], qcy[kQ];
   const double stw = a.scal[6] * 0.6180339887498949;  // Weyl step phase
   const float sph = (float)(stw - floor(stw));
   const float dsc0 = a.dither ? 0x1p-23f : 0.f, dsc1 = a.dither ? -0x1p-24f : 0.f;
+  const bool anyin = __ballot(s.mask != 0) != 0;
   const T* fe = a.fcur + 3 * (size_t)e;
+  // prime the queue: f of v0 .. v0+kDepth-1, and the first ordinate's row
+  T q[kQ][3];
 #pragma unroll
   for (int j = 0; j < kQ; ++j) {
-    q[j][0] = q[j][1] = q[j][2] = qx[j] = qy[j] = qi[j] = T(0);
-    qp[j] = 0.f;
-    qw[j] = qcx[j] = qcy[j] = 0.0;
+    q[j][0] = q[j][1] = q[j][2] = T(0);
     if (j < kDepth) {  // slots without an element read element 0
-      const int v = min(v0 + j, v1 - 1);
-      const T* fp = fe + (size_t)v * a.ldf;
+      const T* fp = fe + (size_t)min(v0 + j, v1 - 1) * a.ldf;
       q[j][0] = fp[0];
       q[j][1] = fp[1];
       q[j][2] = fp[2];
-      qx[j] = ldc(a.vtab, v);
-      qy[j] = ldc(a.vtab, V + v);
-      qi[j] = ldc(a.vtab, 2 * V + v);
-      qp[j] = sph + (float)ldc(a.vtab, 3 * V + v);
-      if (kMom) {
-        qw[j] = ldc(a.vtd, 4 * V + v);
-        qcx[j] = ldc(a.vtd, 5 * V + v);
-        qcy[j] = ldc(a.vtd, 6 * V + v);
-      }
     }
   }
+  OrdRow<T> row = ord_row<T, kMom>(a.vrow, v0);
   double m0[3] = {0, 0, 0}, m1[3] = {0, 0, 0}, m2[3] = {0, 0, 0};
   for (int vb = v0; vb < v1; vb += kQ) {
 #pragma unroll
@@ -521,25 +582,18 @@ k_update(UpdArgs<T> a) {
       if (v < v1) {  // uniform over the block
         // unconditional (clamped at the chunk's last ordinate), so the load
         // lands in its slot without a branch that would force a wait
-        const int vn = min(v + kDepth, v1 - 1);
+        const T* fp = fe + (size_t)min(v + kDepth, v1 - 1) * a.ldf;
         const int jn = (j + kDepth) % kQ;
-        {
-          const T* fp = fe + (size_t)vn * a.ldf;
-          q[jn][0] = fp[0];
-          q[jn][1] = fp[1];
-          q[jn][2] = fp[2];
-          qx[jn] = ldc(a.vtab, vn);
-          qy[jn] = ldc(a.vtab, V + vn);
-          qi[jn] = ldc(a.vtab, 2 * V + vn);
-          qp[jn] = sph + (float)ldc(a.vtab, 3 * V + vn);
-          if (kMom) {
-            qw[jn] = ldc(a.vtd, 4 * V + vn);
-            qcx[jn] = ldc(a.vtd, 5 * V + vn);
-            qcy[jn] = ldc(a.vtd, 6 * V + vn);
-          }
-        }
-        update_ordinate<T, kMom, kCM>(a, s, v, qx[j], qy[j], qi[j], qp[j], dsc0, dsc1, q[j], s_f[j], dte,
-                                 res, chg, qw[j], qcx[j], qcy[j], m0, m1, m2);
+        q[jn][0] = fp[0];
+        q[jn][1] = fp[1];
+        q[jn][2] = fp[2];
+        Half<T> hf = update_first<T>(s, row.ux, row.uy, q[j], s_f[j], dte);
+        __syncthreads();  // the one barrier per ordinate
+        const OrdRow<T> cur = row;
+        row = ord_row<T, kMom>(a.vrow, min(v + 1, v1 - 1));
+        if (s.owned)
+          update_second<T, kMom, kCM>(a, s, hf, v, cur, sph + (float)cur.ph, dsc0, dsc1, anyin,
+                                      q[j], s_f[j], res, chg, m0, m1, m2);
       }
     }
   }
@@ -1342,7 +1396,7 @@ struct Ctx {
   int cur = 0;
   void *geo = nullptr, *enx = nullptr, *eny = nullptr, *ealen = nullptr, *np = nullptr,
        *unx = nullptr, *uny = nullptr,
-       *vtab = nullptr, *refl_t = nullptr, *wpart = nullptr;
+       *vtab = nullptr, *vrow = nullptr, *refl_t = nullptr, *wpart = nullptr;
   int *einfo = nullptr, *eslot = nullptr, *emask = nullptr, *ewslot = nullptr, *uinfo = nullptr,
       *refl_i = nullptr, *wall_bside = nullptr, *tiles = nullptr, *halo = nullptr,
       *wall_elems = nullptr, *eta_side = nullptr, *fside = nullptr, *pt_ptr = nullptr,
@@ -1538,8 +1592,8 @@ int step_once(Ctx& c) {
   UpdArgs<T> u;
   u.fcur = fc; u.fnxt = fn; u.geo = (const T*)c.geo; u.uinfo = c.uinfo;
   u.unx = (const T*)c.unx; u.uny = (const T*)c.uny;
-  u.emask = c.emask; u.ewslot = c.ewslot; u.np = (const T*)c.np; u.vtab = (const T*)c.vtab;
-  u.tiles = c.tiles; u.halo = c.halo; u.wpart = (T*)c.wpart; u.vtd = c.vtd; u.msum = c.msum;
+  u.emask = c.emask; u.ewslot = c.ewslot; u.np = (const T*)c.np; u.vrow = (const T*)c.vrow;
+  u.tiles = c.tiles; u.halo = c.halo; u.wpart = (T*)c.wpart; u.msum = c.msum;
   u.scal = c.scal; u.res_part = c.res_part; u.res_stride = c.nblk_upd + c.nblk_wall;
   u.E = p.E; u.V = p.V; u.ntiles = c.ntiles; u.vchunk = c.vchunk;
   u.ephase = c.ephase;
@@ -1701,7 +1755,7 @@ int upload_tables(Ctx& c) {
       uny[i] = flux ? (T)(sg * ed.alen * ed.ny) : T(0);
       if (ed.kind == kInterior) {
         const int nbk = ed.sign > 0 ? ed.b1 : ed.b2, nbk1 = ed.sign > 0 ? ed.b2 : ed.b1;
-        uinfo[i] = (nbk << kUpdNbK) | (nbk1 << kUpdNbK1) | (ed.sign > 0 ? 0 : kUpdRight) |
+        uinfo[i] = (nbk << kUpdNbK) | (nbk1 << kUpdNbK1) |
                    (p.nbr_slot[3 * (size_t)e + k] << kUpdSlot);
       } else {
         uinfo[i] = kUpdOwn | (ed.kind == kInflow ? kUpdInflow : 0);
@@ -1742,7 +1796,17 @@ int upload_tables(Ctx& c) {
     // the FP32-bulk pressure sum's weight: 0.5 w |c_b|^2
     vtd[7 * V + v] = 0.5 * p.wv[v] * (p.cxb[v] * p.cxb[v] + p.cyb[v] * p.cyb[v]);
   }
+  // the same, one kOrdRow-byte row per ordinate: the update kernel's scalars
+  // in two scalar loads instead of seven
+  std::vector<T> vrow((size_t)V * (kOrdRow / sizeof(T)), T(0));
+  for (int v = 0; v < V; ++v) {
+    T* r = &vrow[(size_t)v * (kOrdRow / sizeof(T))];
+    for (int k = 0; k < 4; ++k) r[k] = vtab[(size_t)k * V + v];
+    const double m[3] = {vtd[4 * (size_t)V + v], vtd[5 * (size_t)V + v], vtd[6 * (size_t)V + v]};
+    std::memcpy(r + 4, m, sizeof(m));
+  }
   if ((st = upload((T**)&c.vtab, vtab, c.owned))) return st;
+  if ((st = upload((T**)&c.vrow, vrow, c.owned))) return st;
   if ((st = upload(&c.vtd, vtd, c.owned))) return st;
   const size_t NW = p.wall_sides.size();
   std::vector<int> ri(2 * NW * V);
@@ -1984,11 +2048,14 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   c.gs = prm->order == DGBGK_ORDER_REFERENCE ? 1 : 0;
   if (const char* ng = std::getenv("DGBGK_NO_GRAPH")) c.use_graph = ng[0] == '0';
   c.tsz = c.prec ? 4 : 8;
-  // ordinates of f in flight per update thread beyond the one computed:
-  // one (a second costs a wavefront of occupancy in both forms: FP64 3 -> 2,
-  // FP32 5 -> 4 per SIMD; measured 6% slower in FP32 at 1M triangles), and
-  // whether the update kernel also sums the first moment pass
-  c.depth = 1;
+  // ordinates of f in flight per update thread beyond the one computed, and
+  // whether the update kernel also sums the first moment pass.  FP32: two (96
+  // registers, as many wavefronts per SIMD as with one: update 306 -> 298 us
+  // at 101,753 x 512, 326 -> 314 us at 25,781 x 2048, 11.60 -> 11.36 ms at
+  // 1,005,669 x 2048) where the chip's 256 x 5 resident blocks walk 16
+  // ordinates each or more; shorter chunks gain nothing from it (21.1 against
+  // 21.3 us at 5,763 x 128).  FP64: one (629 -> 636 us with two).
+  c.depth = c.prec && prm->immat != 0 && c.p.tile_e0.size() * (size_t)c.p.V >= 16 * 256 * 5 ? 2 : 1;
   if (const char* pd = std::getenv("DGBGK_PREFETCH")) {
     const int d = std::atoi(pd);
     if (d >= 1 && d <= 2 && prm->immat != 0) c.depth = d;  // IMMAT = 0: depth 1 only

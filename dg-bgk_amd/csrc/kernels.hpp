@@ -17,6 +17,8 @@
 //   np       T[5][3E]   per node: n*beta2/pi, beta2, u, v, mu (GTEQNF/COMPMU)
 //   vtab     T[4][V]    ordinate velocity (ADVNCE form), inflow value, and
 //                       the FP32 store dither's ordinate phase
+//   vrow     [V] rows of kOrdRow bytes: vtab's four values as T, then the
+//                       moment weights w, w cx, w cy as double
 //   mom      double[5][3E] DISND, DISUX, DISUY, DISPS, MU
 #pragma once
 
@@ -25,6 +27,7 @@
 namespace dgbgk {
 
 constexpr int kSlots = 256;  // LDS slots (= threads) per update block
+constexpr size_t kOrdRow = 64;  // bytes of an ordinate's row of vrow
 
 // einfo bit fields
 __host__ __device__ constexpr int einfo_pack(int kind, int a1, int a2, int b1, int b2,
@@ -37,12 +40,10 @@ struct StepRec {  // same layout as dgbgk_step_info
 };
 
 // Update-kernel edge word (uinfo), one per element edge k (local nodes k,
-// k1 = (k+1)%3): the flux source when the neighbour is upwind and the
-// tie rule of the side's orientation.
+// k1 = (k+1)%3): the flux source when the neighbour is upwind.
 constexpr int kUpdNbK = 0;      // bits 0-1: neighbour's local node at node k
 constexpr int kUpdNbK1 = 2;     // bits 2-3: neighbour's local node at node k1
-constexpr int kUpdRight = 1 << 4;  // this element is the side's right element
-constexpr int kUpdOwn = 1 << 5;    // boundary side: own values are always upwind
+constexpr int kUpdOwn = 1 << 5;    // boundary side: the own element's values
 constexpr int kUpdInflow = 1 << 6; // inflow side: upwind values are zero (FP32 form)
 constexpr int kUpdSlot = 8;     // bits 8+: neighbour's LDS slot
 
@@ -57,11 +58,10 @@ struct UpdArgs {
   const int* __restrict__ emask;   // inflow bits 0..2
   const int* __restrict__ ewslot;  // wall element slot or -1
   const T* __restrict__ np;
-  const T* __restrict__ vtab;
+  const T* __restrict__ vrow;      // [V] rows: see above
   const int* __restrict__ tiles;   // [ntiles][4] e0, nown, hoff, nhalo
   const int* __restrict__ halo;
   T* __restrict__ wpart;           // [NWE][V][8] partial RHS (3), COLL (3), U
-  const double* __restrict__ vtd;  // [8][V]: cxa, cya, cxb, cyb, wv, wv cxb, wv cyb, ...
   double* __restrict__ msum;       // [nvchunks][3][3E] moment partials of f^{k+1}
   const double* __restrict__ scal; // [0] = DTE
   double* __restrict__ res_part;   // per block: max|increment|; +res_stride: max|change|
