@@ -5,8 +5,8 @@
 //   k_eta      FLUCON2 wall mass-flux parameter per type-4 side
 //   k_update   all ordinates of all elements: GTEQNF + GETELC + EDGFLXOPT +
 //              GETINC + ADTHEM + INFLOW, element tiles staged in LDS
-//   k_wall     in-place sweep order: reflected wall fluxes, ordinate by
-//              ordinate per (wall element, speed ring)
+//   k_wall or  in-place sweep order: reflected wall fluxes, every ordinate once
+//   k_wall_ring  what its reflections read is advanced
 //   k_moments  MACROS + COMPMU on f^{k+1}: FP64 compensated sums
 //   k_points   point averages (GETMAC) when the reference gathers them
 //   k_final    residual max, mass, forces, next DTE (ALOTIM2)
@@ -613,38 +613,27 @@ k_update(UpdArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// k_wall: the wall sides of the wall elements, and their update.  Per
-// ordinate, a wall side's flux is the interior form on the element's own
+// k_wall, k_wall_ring: the wall sides of the wall elements, and their update.
+// Per ordinate, a wall side's flux is the interior form on the element's own
 // values when c.n >= 0 (src/getbou.f90:174-187), else the reflected
 // distribution (src/getbou.f90:190-255).  In the reference's in-place
 // velocity sweep the reflection reads f at ordinates I1, I2 of the same
 // element, and those already advanced this step (index < v) are read from
 // the new buffer (src/getbou.f90:245-250 inside src/advnce.f90:273-383);
-// with jacobi set every read is from the previous step.  One thread per
-// (wall element, speed ring) when every reflection stays in its ring, else
-// per wall element over all ordinates.
+// with jacobi set every read is from the previous step.
 // ---------------------------------------------------------------------------
+
+// A wall element: its edges, lumped mass, inflow nodes and dither phases.
 template <typename T>
-__global__ void __launch_bounds__(256) k_wall(WallArgs<T> a) {
-  __shared__ double s_red[8];
-  // per thread, the ring's freshly advanced f (when reflections stay in the
-  // ring): the in-place reads of ordinates < v come from LDS
-  extern __shared__ unsigned char s_dyn[];
-  T* s_ring = reinterpret_cast<T*>(s_dyn) + (size_t)threadIdx.x * 3 * a.T_;
-  const bool use_lds = a.lds_ring;
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  double res = 0.0, chg = 0.0;
-  if (gid < a.nwe * a.ngroups) {
-    const int we = gid / a.ngroups, grp = gid % a.ngroups;
-    const int e = a.wall_elems[we];
-    const int E = a.E, V = a.V;
-    const size_t N3 = 3 * (size_t)E;
-    const int vb = grp * a.gsize;
-    const int ve = vb + a.gsize;
-    const T dte = (T)a.scal[0];
-    const T mdt = a.geo[7 * E + e] * dte;
-    int info[3], nsl[3];
-    T enx[3], eny[3], eal[3];
+struct WallElem {
+  int e, we, mask, info[3], nsl[3];
+  T enx[3], eny[3], eal[3], mdt;
+  float wph, sph;
+  __device__ __forceinline__ WallElem(const WallArgs<T>& a, int w) {
+    we = w;
+    e = a.wall_elems[w];
+    const int E = a.E;
+    mdt = a.geo[7 * E + e] * (T)a.scal[0];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       info[k] = a.einfo[k * E + e];
@@ -653,42 +642,114 @@ __global__ void __launch_bounds__(256) k_wall(WallArgs<T> a) {
       eny[k] = a.eny[k * E + e];
       eal[k] = a.ealen[k * E + e];
     }
-    const int mask = a.emask[e];
-    const T alpha = a.alpha;
-    // FP32 store dither (as in k_update): node, ordinate and step phases
-    const float wph = a.ephase[e];
+    mask = a.emask[e];
+    // FP32 store dither (as in k_update): element, ordinate and step phases
+    wph = a.ephase[e];
     const double stw = a.scal[6] * 0.6180339887498949;
-    const float sph = (float)(stw - floor(stw));
-    for (int v = vb; v < ve; ++v) {
-      const T* wp = a.wpart + ((size_t)we * V + v) * 8;
-      T rhs[3] = {wp[0], wp[1], wp[2]};
-      const T cold[3] = {wp[3], wp[4], wp[5]};  // collision term times DTE
-      const T U = wp[6];
-      const T ux = a.vtab[v], uy = a.vtab[V + v];
-      const T* fc = a.fcur + (size_t)v * a.ldf + 3 * (size_t)e;
-      const T f[3] = {fc[0], fc[1], fc[2]};
-      // FP32: the edge terms act on (g - gbar), as in k_update's FP32 form
-      // (the element's own values as differences from f_0)
-      T hw[3] = {T(0), T(0), T(0)}, gbar = T(0);
-      if constexpr (sizeof(T) == 4) {
-        const T d1 = f[1] - f[0], d2 = f[2] - f[0];
-        const T db = (T(1) / T(3)) * (d1 + d2);
-        hw[0] = -db;
-        hw[1] = d1 - db;
-        hw[2] = d2 - db;
-        gbar = (f[0] + db) - U;
+    sph = (float)(stw - floor(stw));
+  }
+};
+
+// One ordinate of one wall element, but for the values its reflections read.
+template <typename T>
+struct WallOrd {
+  T rhs[3], cold[3], U, f[3], ux, uy;
+  T hw[3], gbar;  // FP32: the edge terms act on (g - gbar), as in k_update's
+                  // FP32 form (the element's own values as differences from f_0)
+  __device__ __forceinline__ WallOrd(const WallArgs<T>& a, const WallElem<T>& w, int v) {
+    const T* wp = a.wpart + ((size_t)w.we * a.V + v) * 8;
+    const T* fc = a.fcur + (size_t)v * a.ldf + 3 * (size_t)w.e;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      rhs[k] = wp[k];
+      cold[k] = wp[3 + k];  // collision term times DTE
+      f[k] = fc[k];
+      hw[k] = T(0);
+    }
+    U = wp[6];
+    ux = a.vtab[v];
+    uy = a.vtab[a.V + v];
+    gbar = T(0);
+    if constexpr (sizeof(T) == 4) {
+      // which products are fused is written out, so that every form of the
+      // pass rounds alike (left to the compiler it depends on the code around)
+      const T c13 = T(1) / T(3), d1 = f[1] - f[0], d2 = f[2] - f[0], sum = d1 + d2;
+      T db = c13 * sum;
+      asm("" : "+v"(db));
+      hw[0] = -db;
+      hw[1] = fma(-c13, sum, d1);
+      hw[2] = d2 - db;
+      gbar = fma(c13, sum, f[0]) - U;
+    }
+  }
+  // adds side k's flux: leaving (own values) or the distribution g1, g2
+  // entering at the side's two nodes
+  __device__ __forceinline__ void side(const WallElem<T>& w, int k, bool leaving, T g1, T g2) {
+    const int a1 = k, a2 = (k + 1) % 3;  // boundary side: (p1, p2) = (k, k+1)
+    if (leaving) {
+      g1 = sizeof(T) == 4 ? hw[a1] : f[a1] - U;
+      g2 = sizeof(T) == 4 ? hw[a2] : f[a2] - U;
+    } else if constexpr (sizeof(T) == 4) {
+      g1 = g1 - gbar;
+      g2 = g2 - gbar;
+    }
+    T r1, r2;
+    edge_rhsi(ux, uy, w.enx[k], w.eny[k], w.eal[k], g1, g2, r1, r2);
+    rhs[a1] += r1;
+    rhs[a2] += r2;
+  }
+  // increment, clamp and inflow reset into fn and the new buffer
+  __device__ __forceinline__ void finish(const WallArgs<T>& a, const WallElem<T>& w, int v,
+                                         T (&fn)[3], double& res, double& chg) {
+    T* fo = a.fnxt + (size_t)v * a.ldf + 3 * (size_t)w.e;
+    const T fin = a.vtab[2 * a.V + v];
+    const float ph = w.sph + (float)a.vtab[3 * a.V + v];
+    const float wt = fmaf(__builtin_amdgcn_fractf(w.wph + ph), a.dither ? 0x1p-23f : 0.f,
+                          a.dither ? -0x1p-24f : 0.f);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const T d = node_increment(a.cmminc != 0, w.mdt, rhs[k], cold[k], res);
+      T dk = d;
+      if constexpr (sizeof(T) == 4)
+        dk = fmaf(wt, __uint_as_float(__float_as_uint(f[k]) & 0x7f800000u), dk);
+      T x = f[k] + dk;
+      x = x < T(0) ? T(0) : x;
+      if ((w.mask >> k) & 1) x = fin;
+      T cg = fabs(x - f[k]);
+      if constexpr (sizeof(T) == 4) {  // the increment, as in k_update
+        if (x != T(0) && !((w.mask >> k) & 1)) cg = fabs(d);
       }
+      chg = fmax(chg, (double)cg);
+      fo[k] = x;
+      fn[k] = x;
+    }
+  }
+};
+
+// One thread per (wall element, group of gsize ordinates): every ordinate by
+// itself where nothing is read in place, else all ordinates of the element
+// in order (rings longer than a block, or reflections that leave their ring).
+template <typename T>
+__global__ void __launch_bounds__(256) k_wall(WallArgs<T> a) {
+  __shared__ double s_red[8];
+  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+  double res = 0.0, chg = 0.0;
+  if (gid < a.nwe * a.ngroups) {
+    const WallElem<T> w(a, gid / a.ngroups);
+    const int e = w.e, V = a.V;
+    const int vb = (gid % a.ngroups) * a.gsize;
+    const T alpha = a.alpha;
+    for (int v = vb; v < vb + a.gsize; ++v) {
+      WallOrd<T> o(a, w, v);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        if ((info[k] & 3) != 3) continue;
-        const int a1 = k, a2 = (k + 1) % 3;  // boundary side: (p1, p2) = (k, k+1)
-        const int ws = nsl[k];
+        if ((w.info[k] & 3) != 3) continue;
+        const int a1 = k, a2 = (k + 1) % 3;
+        const int ws = w.nsl[k];
         const size_t rk = (size_t)ws * V + v;
         const int i1 = a.refl_i[2 * rk];
-        T g1, g2;
+        T g1 = T(0), g2 = T(0);
         if (i1 < 0) {  // molecules leaving through the wall: own values
-          g1 = f[a1] - U;
-          g2 = f[a2] - U;
         } else if (a.diffuse) {  // alpha = 1: (1 - alpha) * Rf is exactly 0
           const T mf = a.refl_t[3 * rk + 2] * (T)a.eta[a.wall_bside[ws]];
           g1 = alpha * mf;
@@ -697,62 +758,116 @@ __global__ void __launch_bounds__(256) k_wall(WallArgs<T> a) {
           const int i2 = a.refl_i[2 * rk + 1];
           const T zd1 = a.refl_t[3 * rk], zd2 = a.refl_t[3 * rk + 1];
           const T mw = a.refl_t[3 * rk + 2];
-          const T* s1;
-          const T* s2;
-          if (use_lds) {
-            s1 = i1 < v ? s_ring + 3 * (i1 - vb) : a.fcur + (size_t)i1 * a.ldf + 3 * (size_t)e;
-            s2 = i2 < v ? s_ring + 3 * (i2 - vb) : a.fcur + (size_t)i2 * a.ldf + 3 * (size_t)e;
-          } else if (a.jacobi) {
-            s1 = a.fcur + (size_t)i1 * a.ldf + 3 * (size_t)e;
-            s2 = a.fcur + (size_t)i2 * a.ldf + 3 * (size_t)e;
-          } else {
-            s1 = (i1 < v ? a.fnxt : a.fcur) + (size_t)i1 * a.ldf + 3 * (size_t)e;
-            s2 = (i2 < v ? a.fnxt : a.fcur) + (size_t)i2 * a.ldf + 3 * (size_t)e;
-          }
+          const T* s1 = (!a.jacobi && i1 < v ? a.fnxt : a.fcur) + (size_t)i1 * a.ldf + 3 * (size_t)e;
+          const T* s2 = (!a.jacobi && i2 < v ? a.fnxt : a.fcur) + (size_t)i2 * a.ldf + 3 * (size_t)e;
           const T rf1 = (zd2 * s1[a1] + zd1 * s2[a1]) / (zd1 + zd2);
           const T rf2 = (zd2 * s1[a2] + zd1 * s2[a2]) / (zd1 + zd2);
           const T mf = mw * (T)a.eta[a.wall_bside[ws]];
           g1 = (T(1) - alpha) * rf1 + alpha * mf;
           g2 = (T(1) - alpha) * rf2 + alpha * mf;
         }
-        if constexpr (sizeof(T) == 4) {  // FP32 form: g - gbar
-          if (i1 < 0) {
-            g1 = hw[a1];
-            g2 = hw[a2];
-          } else {
-            g1 = g1 - gbar;
-            g2 = g2 - gbar;
-          }
-        }
-        T r1, r2;
-        edge_rhsi(ux, uy, enx[k], eny[k], eal[k], g1, g2, r1, r2);
-        rhs[a1] += r1;
-        rhs[a2] += r2;
+        o.side(w, k, i1 < 0, g1, g2);
       }
-      T* fo = a.fnxt + (size_t)v * a.ldf + 3 * (size_t)e;
-      const T fin = a.vtab[2 * V + v];
-      const float ph = sph + (float)a.vtab[3 * V + v];
-      const float wt = fmaf(__builtin_amdgcn_fractf(wph + ph), a.dither ? 0x1p-23f : 0.f,
-                            a.dither ? -0x1p-24f : 0.f);
+      T fn[3];
+      o.finish(a, w, v, fn, res, chg);
+    }
+  }
+  const double r = block_max(res, s_red);
+  if (threadIdx.x == 0) a.res_part[blockIdx.x] = r;
+  const double rc = block_max(chg, s_red);
+  if (threadIdx.x == 0) a.res_part[a.res_stride + blockIdx.x] = rc;
+}
+
+// The in-place order where every reflection stays in its speed ring: one
+// thread per ordinate, a ring's T threads in one block, 256/T rings per
+// block.  An ordinate waits for the (at most two per side) ordinates of
+// lower index that its reflections read as advanced; a reflection reads
+// ordinates that leave through the wall, which wait for nothing, so two or
+// three rounds finish a ring.  (The lowest unfinished ordinate never waits:
+// at most T rounds.)  Each ordinate's arithmetic and reads are those of the
+// ordered sweep.  One thread walking a ring in order, with its loads in
+// line, took 74 us at 157 wall elements x 16 rings x 32 ordinates and 26 us
+// at 64 x 8 x 16; this takes 12 and 9 us.
+template <typename T>
+__global__ void __launch_bounds__(256) k_wall_ring(WallArgs<T> a) {
+  __shared__ double s_red[8];
+  __shared__ T s_new[256][3];
+  __shared__ int s_done[256], s_left[2];
+  const int nT = a.gsize, tid = threadIdx.x, grp = tid / nT, base = grp * nT;
+  const int pair = blockIdx.x * (256 / nT) + grp;
+  const bool live = grp < 256 / nT && pair < a.nwe * a.ngroups;
+  double res = 0.0, chg = 0.0;
+  // threads without an ordinate (a block's last ones) count as finished and
+  // run the same rounds, on the first pair's data, without storing
+  const int p = live ? pair : 0, v0 = (p % a.ngroups) * nT, v = v0 + (live ? tid - base : 0);
+  bool done = !live;
+  s_done[tid] = done;
+  if (tid < 2) s_left[tid] = 0;
+  const WallElem<T> w(a, p / a.ngroups);
+  WallOrd<T> o(a, w, v);
+  // per side: the bracketing ordinates, their weights, the wall's part, and
+  // what is read from the previous step
+  int i1[3], i2[3];
+  T zd1[3], zd2[3], mf[3], p1[3][2], p2[3][2];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    i1[k] = i2[k] = -1;
+    zd1[k] = zd2[k] = mf[k] = T(0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) p1[k][j] = p2[k][j] = T(0);
+    if ((w.info[k] & 3) != 3) continue;
+    const int ws = w.nsl[k];
+    const size_t rk = (size_t)ws * a.V + v;
+    i1[k] = a.refl_i[2 * rk];
+    if (i1[k] < 0) continue;
+    i2[k] = a.refl_i[2 * rk + 1];
+    zd1[k] = a.refl_t[3 * rk];
+    zd2[k] = a.refl_t[3 * rk + 1];
+    mf[k] = a.refl_t[3 * rk + 2] * (T)a.eta[a.wall_bside[ws]];
+    const T* f1 = a.fcur + (size_t)i1[k] * a.ldf + 3 * (size_t)w.e;
+    const T* f2 = a.fcur + (size_t)i2[k] * a.ldf + 3 * (size_t)w.e;
+    p1[k][0] = f1[k];
+    p1[k][1] = f1[(k + 1) % 3];
+    p2[k][0] = f2[k];
+    p2[k][1] = f2[(k + 1) % 3];
+  }
+  __syncthreads();
+  for (int r = 0;; r ^= 1) {
+    bool ready = !done;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (i1[k] >= 0 && i1[k] < v) ready = ready && s_done[base + i1[k] - v0];
+      if (i2[k] >= 0 && i2[k] < v) ready = ready && s_done[base + i2[k] - v0];
+    }
+    __syncthreads();  // all flags read
+    if (ready) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        const T d = node_increment(a.cmminc != 0, mdt, rhs[k], cold[k], res);
-        T dk = d;
-        if constexpr (sizeof(T) == 4) {
-          dk = fmaf(wt, __uint_as_float(__float_as_uint(f[k]) & 0x7f800000u), dk);
+        if ((w.info[k] & 3) != 3) continue;
+        T g[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int nd = (k + j) % 3;
+          const T x1 = i1[k] >= 0 && i1[k] < v ? s_new[base + i1[k] - v0][nd] : p1[k][j];
+          const T x2 = i2[k] >= 0 && i2[k] < v ? s_new[base + i2[k] - v0][nd] : p2[k][j];
+          const T rf = (zd2[k] * x1 + zd1[k] * x2) / (zd1[k] + zd2[k]);
+          g[j] = (T(1) - a.alpha) * rf + a.alpha * mf[k];
         }
-        T fn = f[k] + dk;
-        fn = fn < T(0) ? T(0) : fn;
-        if ((mask >> k) & 1) fn = fin;
-        T cg = fabs(fn - f[k]);
-        if constexpr (sizeof(T) == 4) {  // the increment, as in k_update
-          if (fn != T(0) && !((mask >> k) & 1)) cg = fabs(d);
-        }
-        chg = fmax(chg, (double)cg);
-        fo[k] = fn;
-        if (use_lds) s_ring[3 * (v - vb) + k] = fn;
+        o.side(w, k, i1[k] < 0, g[0], g[1]);
       }
+      T fn[3];
+      o.finish(a, w, v, fn, res, chg);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) s_new[tid][k] = fn[k];
+      s_done[tid] = 1;
+      done = true;
     }
+    if (!done) s_left[r] = 1;
+    __syncthreads();  // this round's values, flags and count
+    const int left = s_left[r];
+    __syncthreads();
+    if (tid == 0) s_left[r] = 0;  // next written two rounds on
+    if (!left) break;
   }
   const double r = block_max(res, s_red);
   if (threadIdx.x == 0) a.res_part[blockIdx.x] = r;
@@ -1408,8 +1523,7 @@ struct Ctx {
   float* ephase = nullptr;  // [E] FP32 store dither phase per element
   StepRec* rec = nullptr;
   int rec_cap = 0;
-  int wall_tpb = 256;
-  int gsize = 1, wall_diffuse = 0, wall_lds = 0;  // k_wall ordinates per thread, modes
+  int gsize = 1, wall_diffuse = 0, wall_ring = 0;  // wall pass: ordinates per group, modes
   int slots = 256;   // update kernel: tile slots (threads per block)
   int depth = 1;     // update kernel: ordinates of f in flight (1 or 2)
   int fuse_mom = 1;  // update kernel also does the first moment pass
@@ -1617,13 +1731,14 @@ int step_once(Ctx& c) {
     w.ldf = (long long)c.ldf;
     w.dither = c.dither;
     w.cmminc = c.p.prm.immat == 0;
-    w.T_ = p.T; w.ngroups = c.ngroups; w.gsize = c.gsize; w.nwe = (int)p.wall_elems.size();
+    w.ngroups = c.ngroups; w.gsize = c.gsize; w.nwe = (int)p.wall_elems.size();
     w.jacobi = c.gs ? 0 : 1;
     w.diffuse = c.wall_diffuse;
-    w.lds_ring = c.wall_lds;
     tbegin(c, 1);
-    const size_t lds = c.wall_lds ? (size_t)c.wall_tpb * 3 * p.T * sizeof(T) : 0;
-    hipLaunchKernelGGL(k_wall<T>, dim3(c.nblk_wall), dim3(c.wall_tpb), lds, c.stream, w);
+    if (c.wall_ring)
+      hipLaunchKernelGGL(k_wall_ring<T>, dim3(c.nblk_wall), dim3(256), 0, c.stream, w);
+    else
+      hipLaunchKernelGGL(k_wall<T>, dim3(c.nblk_wall), dim3(256), 0, c.stream, w);
     HIPCK(hipGetLastError());
     tend(c, 1);
   }
@@ -2109,29 +2224,26 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   c.nvchunks = (p.V + c.vchunk - 1) / c.vchunk;
   c.nblk_upd = c.ntiles * c.nvchunks;
   const int nwe = (int)p.wall_elems.size();
-  // k_wall: ordinates that depend on each other through in-place reflected
-  // reads are walked by one thread in order.  Without in-place reads
-  // (Jacobi order, or a fully diffuse wall, whose reflected part has weight
-  // 1 - alpha = 0) every (wall element, ordinate) is independent.
-  c.wall_tpb = 256;
+  // The wall pass.  Without in-place reads (Jacobi order, or a fully diffuse
+  // wall, whose reflected part has weight 1 - alpha = 0) every (wall element,
+  // ordinate) is independent.  With them, k_wall_ring takes the rings that
+  // are closed and fit a block; otherwise one thread walks the ordinates
+  // that may depend on each other in order.
   c.wall_diffuse = prm->alpha == 1.0 ? 1 : 0;
-  c.wall_lds = 0;
+  c.wall_ring = 0;
   if (!c.gs || c.wall_diffuse) {
     c.ngroups = p.V;
     c.gsize = 1;
   } else if (p.ring_separable) {
-    // one thread per speed ring; its freshly advanced f is staged in LDS
     c.ngroups = p.R;
     c.gsize = p.T;
-    const size_t per = 3 * (size_t)p.T * c.tsz;
-    while (c.wall_tpb > 64 && (size_t)c.wall_tpb * per > 65536) c.wall_tpb >>= 1;
-    if ((size_t)c.wall_tpb * per <= 65536) c.wall_lds = 1;
-    else c.wall_tpb = 256;
+    c.wall_ring = p.T <= 256 ? 1 : 0;
   } else {
     c.ngroups = 1;
     c.gsize = p.V;
   }
-  c.nblk_wall = nwe ? (nwe * c.ngroups + c.wall_tpb - 1) / c.wall_tpb : 0;
+  const int wall_per = c.wall_ring ? 256 / p.T : 256;  // groups per block
+  c.nblk_wall = nwe ? (nwe * c.ngroups + wall_per - 1) / wall_per : 0;
   // k_moments: one wavefront per 64 nodes leaves fewer than ~8 per SIMD
   // below 512k nodes, and then up to four share each node's ordinates.  The
   // choice depends on the node count only, so a mesh gives the same sums

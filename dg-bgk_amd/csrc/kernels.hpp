@@ -96,10 +96,9 @@ struct WallArgs {
   const float* __restrict__ ephase; // [E] FP32 store dither phase per element
   int res_stride;
   T alpha;
-  int E, V, T_, ngroups, gsize, nwe;  // ngroups threads per wall element, gsize ordinates each
+  int E, V, ngroups, gsize, nwe;  // ngroups groups of gsize ordinates per wall element
   int jacobi;    // reflections read f of the previous step only
   int diffuse;   // alpha = 1: the reflected part has weight 0 and is not read
-  int lds_ring;  // one thread per speed ring, in-place reads staged in LDS
   long long ldf;  // row stride of f
   int dither;     // FP32: dithered (unbiased) rounding of the f store
   int cmminc;     // IMMAT = 0: as in UpdArgs
