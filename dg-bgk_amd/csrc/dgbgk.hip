@@ -7,7 +7,8 @@
 //              GETINC + ADTHEM + INFLOW, element tiles staged in LDS
 //   k_wall or  in-place sweep order: reflected wall fluxes, every ordinate once
 //   k_wall_ring  what its reflections read is advanced
-//   k_moments  MACROS + COMPMU on f^{k+1}: FP64 compensated sums
+//   k_moments or MACROS + COMPMU on f^{k+1}: FP64 sums
+//   k_moments_once
 //   k_points   point averages (GETMAC) when the reference gathers them
 //   k_final    residual max, mass, forces, next DTE (ALOTIM2)
 #include <hip/hip_runtime.h>
@@ -897,6 +898,38 @@ __global__ void __launch_bounds__(256) k_wall_ring(WallArgs<T> a) {
 template <typename T>
 constexpr int kMomRing = sizeof(T) == 4 ? DGBGK_MOM_RING32 : DGBGK_MOM_RING64;
 
+// A node's fields and next-step parameters from its sums: n, the mean
+// velocity, the pressure and relative-speed sums.
+template <typename T>
+__device__ __forceinline__ void node_result(const MomArgs<T>& a, size_t k, double n, double ux,
+                                            double uy, double sp, double st, double& mu,
+                                            double& mass) {
+  constexpr bool kComp = sizeof(T) < sizeof(double);
+  const size_t N3 = 3 * (size_t)a.E;
+  const bool dens = n >= 1e-20;
+  const double nd = dens ? n : 0.0;
+  const double ps = (sp - (kComp ? 0.5 * nd * (ux * ux + uy * uy) : 0.0)) * a.mm;
+  const double ctv = dens ? st / n : 0.0;
+  mu = sqrt(2.0) * ctv * a.sigt * nd;
+  a.mom[k] = nd;
+  a.mom[N3 + k] = ux;
+  a.mom[2 * N3 + k] = uy;
+  a.mom[3 * N3 + k] = ps;
+  a.mom[4 * N3 + k] = mu;
+  // GTEQNF parameters (src/gteqnf.f90:28-37)
+  double pa = 0.0, pb = 0.0;
+  if (!(ps < 1e-20)) {
+    pb = (a.mm * nd) / (2 * ps);
+    pa = nd * (pb / 3.1416);
+  }
+  a.np[k] = (T)pa;
+  a.np[N3 + k] = (T)pb;
+  a.np[2 * N3 + k] = (T)ux;
+  a.np[3 * N3 + k] = (T)uy;
+  a.np[4 * N3 + k] = (T)mu;
+  mass = nd * a.rj[k / 3] / 6.0;
+}
+
 template <typename T, int S>
 __global__ void __launch_bounds__(256) k_moments(MomArgs<T> a) {
   constexpr bool kComp = sizeof(T) < sizeof(double);
@@ -986,9 +1019,8 @@ __global__ void __launch_bounds__(256) k_moments(MomArgs<T> a) {
     }
   }
   const double n = t0 - e0;
-  double nd = 0.0, ux = 0.0, uy = 0.0;
+  double ux = 0.0, uy = 0.0;
   if (n >= 1e-20) {
-    nd = n;
     ux = (t1 - e1) / n;
     uy = (t2 - e2s) / n;
   }
@@ -1097,32 +1129,126 @@ __global__ void __launch_bounds__(256) k_moments(MomArgs<T> a) {
     }
   }
   double mu = 0.0, mass = 0.0;
-  if (sub == 0 && live) {
-    const double ps = ((tp - ep) - (kComp ? 0.5 * nd * (ux * ux + uy * uy) : 0.0)) * a.mm;
-    const double ctv = dens ? (tt - et) / n : 0.0;
-    mu = sqrt(2.0) * ctv * a.sigt * nd;
-    a.mom[k] = nd;
-    a.mom[N3 + k] = ux;
-    a.mom[2 * N3 + k] = uy;
-    a.mom[3 * N3 + k] = ps;
-    a.mom[4 * N3 + k] = mu;
-    // GTEQNF parameters (src/gteqnf.f90:28-37)
-    double pa = 0.0, pb = 0.0;
-    if (!(ps < 1e-20)) {
-      pb = (a.mm * nd) / (2 * ps);
-      pa = nd * (pb / 3.1416);
-    }
-    a.np[k] = (T)pa;
-    a.np[N3 + k] = (T)pb;
-    a.np[2 * N3 + k] = (T)ux;
-    a.np[3 * N3 + k] = (T)uy;
-    a.np[4 * N3 + k] = (T)mu;
-    mass = nd * a.rj[k / 3] / 6.0;
-  }
+  if (sub == 0 && live) node_result(a, k, n, ux, uy, tp - ep, tt - et, mu, mass);
   const double m1 = block_max(mu, s_red);
   if (threadIdx.x == 0) a.mu_part[blockIdx.x] = m1;
   const double m2 = block_sum(mass, s_red);
   if (threadIdx.x == 0) a.mass_part[blockIdx.x] = m2;
+}
+
+// k_moments_once: the same sums where a block's wavefronts hold all V
+// ordinates of 64 nodes in registers (at most kMomHold each), so f is read
+// once, the update leaves no partial sums, and every load of the kernel is
+// in flight at the start.  For meshes whose step is bound by latency:
+// k_moments' rounds of loads (the update's sums, then f) take 26 us at 1,679
+// triangles x 128 in FP64 and 21 us at 5,763 x 128, this 10 and 14, and the
+// update 11 and 18 us against 15 and 21 with its sums.
+constexpr int kMomHold = 32;
+
+template <typename T, int S>
+__global__ void __launch_bounds__(64 * S) k_moments_once(MomArgs<T> a) {
+  constexpr bool kComp = sizeof(T) < sizeof(double);
+  __shared__ double s_part[S][3][64];
+  const int lane = threadIdx.x & 63;
+  const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t N3 = 3 * (size_t)a.E, k = (size_t)blockIdx.x * 64 + lane;
+  const bool live = k < N3;
+  const int V = a.V, vper = (V + S - 1) / S;
+  const int vb = min(V, sub * vper), cnt = min(V, vb + vper) - vb;
+  const T* fp = a.f + (live ? k : 0);
+  T f[kMomHold];
+#pragma unroll
+  for (int j = 0; j < kMomHold; j += 4)  // past the share: its last ordinate, unused
+    if (j < cnt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        f[j + i] = fload_nt(fp + (size_t)(vb + min(j + i, cnt - 1)) * a.ldf);
+    }
+  const double* cxa = a.vtd + vb;
+  const double* cya = a.vtd + V + vb;
+  const double* cxb = a.vtd + 2 * V + vb;
+  const double* cyb = a.vtd + 3 * V + vb;
+  const double* wv = a.vtd + 4 * V + vb;
+  const double* wcx = a.vtd + 5 * V + vb;
+  const double* wcy = a.vtd + 6 * V + vb;
+  const double* hv = a.vtd + 7 * V + vb;
+  const T* vt = a.vtab + vb;
+  // in runs of four ordinates (one set of scalar loads), then one by one
+  auto each = [&](auto&& body) {
+#pragma unroll
+    for (int j = 0; j < kMomHold; j += 4) {
+      if (j + 4 <= cnt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) body(j + i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          if (j + i < cnt) body(j + i);
+      }
+    }
+  };
+  double b0 = 0, b1 = 0, b2 = 0;
+  each([&](int j) {
+    const double fd = (double)f[j];
+    b0 = fma(ldc(wv, j), fd, b0);
+    b1 = fma(ldc(wcx, j), fd, b1);
+    b2 = fma(ldc(wcy, j), fd, b2);
+  });
+  s_part[sub][0][lane] = b0;
+  s_part[sub][1][lane] = b1;
+  s_part[sub][2][lane] = b2;
+  __syncthreads();
+  double t0 = 0, e0 = 0, t1 = 0, e1 = 0, t2 = 0, e2 = 0;
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    nsum<kComp>(t0, e0, s_part[i][0][lane]);
+    nsum<kComp>(t1, e1, s_part[i][1][lane]);
+    nsum<kComp>(t2, e2, s_part[i][2][lane]);
+  }
+  const double n = t0 - e0;
+  const bool dens = n >= 1e-20;
+  const double ux = dens ? (t1 - e1) / n : 0.0, uy = dens ? (t2 - e2) / n : 0.0;
+  const float uxf = (float)ux, uyf = (float)uy;
+  double bp = 0, bt = 0;  // the terms of k_moments' second pass
+  each([&](int j) {
+    if constexpr (kComp) {
+      const float ex = uxf - (float)ldc(vt, j), ey = uyf - (float)ldc(vt + V, j);
+      const float rel = __builtin_amdgcn_sqrtf(fmaf(ex, ex, ey * ey));
+      bp = fma((double)f[j], ldc(hv, j), bp);
+      bt = fma((double)(rel * (float)f[j]), ldc(wv, j), bt);
+    } else {
+      const double fw = (double)f[j] * ldc(wv, j);
+      const double dx = ldc(cxb, j) - ux, dy = ldc(cyb, j) - uy;
+      const double ex = ux - ldc(cxa, j), ey = uy - ldc(cya, j);
+      bp += 0.5 * (dx * dx + dy * dy) * fw;
+      bt += sqrt(ex * ex + ey * ey) * fw;
+    }
+  });
+  __syncthreads();  // every wavefront has read the first sums
+  s_part[sub][0][lane] = bp;
+  s_part[sub][1][lane] = bt;
+  __syncthreads();
+  double mu = 0.0, mass = 0.0;
+  if (sub == 0 && live) {
+    double tp = 0, ep = 0, tt = 0, et = 0;
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      nsum<kComp>(tp, ep, s_part[i][0][lane]);
+      nsum<kComp>(tt, et, s_part[i][1][lane]);
+    }
+    node_result(a, k, n, ux, uy, tp - ep, tt - et, mu, mass);
+  }
+  // only the first wavefront holds results
+  if (sub == 0) {
+    for (int o = 32; o > 0; o >>= 1) {
+      mu = fmax(mu, __shfl_down(mu, o, 64));
+      mass += __shfl_down(mass, o, 64);
+    }
+    if (lane == 0) {
+      a.mu_part[blockIdx.x] = mu;
+      a.mass_part[blockIdx.x] = mass;
+    }
+  }
 }
 
 // FLUCON2 (src/flucon2.f90:133-233): one block per type-4 wall side.
@@ -1528,7 +1654,8 @@ struct Ctx {
   int depth = 1;     // update kernel: ordinates of f in flight (1 or 2)
   int fuse_mom = 1;  // update kernel also does the first moment pass
   int dither = 1;    // FP32 bulk: unbiased (dithered) rounding of the f store
-  int mom_split = 1; // k_moments wavefronts per node (1, 2 or 4)
+  int mom_split = 1; // moments kernel: wavefronts per node
+  int mom_once = 0;  // k_moments_once
   int ntiles = 0, vchunk = 1, nvchunks = 1, nblk_upd = 0, nblk_wall = 0, ngroups = 1,
       nblk_mom = 0, neta = 0, nforce = 0;
   int itime = 0;
@@ -1569,7 +1696,13 @@ int launch_moments(Ctx& c, bool partials = false) {
   m.E = c.p.E;
   m.ldf = (long long)c.ldf;
   m.V = c.p.V;
-  if (c.mom_split == 4)
+  if (c.mom_once && c.mom_split == 4)
+    hipLaunchKernelGGL((k_moments_once<T, 4>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
+  else if (c.mom_once && c.mom_split == 8)
+    hipLaunchKernelGGL((k_moments_once<T, 8>), dim3(c.nblk_mom), dim3(512), 0, c.stream, m);
+  else if (c.mom_once)
+    hipLaunchKernelGGL((k_moments_once<T, 16>), dim3(c.nblk_mom), dim3(1024), 0, c.stream, m);
+  else if (c.mom_split == 4)
     hipLaunchKernelGGL((k_moments<T, 4>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
   else if (c.mom_split == 2)
     hipLaunchKernelGGL((k_moments<T, 2>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
@@ -2176,6 +2309,24 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
     if (d >= 1 && d <= 2 && prm->immat != 0) c.depth = d;  // IMMAT = 0: depth 1 only
   }
   if (const char* fm = std::getenv("DGBGK_FUSE_MOMENTS")) c.fuse_mom = fm[0] != '0';
+  // Moments by k_moments_once (and no sums in the update) while its blocks
+  // of S wavefronts come in about two rounds of the chip or fewer: S the
+  // fewest that hold V ordinates, at most 8192 wavefronts in FP64 and 16384
+  // in FP32 (half the registers, so twice the blocks resident).  Update plus
+  // moments, us, with sums -> without: 1,679 x 128 FP64 41 -> 22, FP32 38 ->
+  // 19; 5,763 x 512 97 -> 85, 77 -> 52; 10,820 x 512 (8112 wavefronts) 133
+  // -> 126, 91 -> 69; 21,178 x 512 (15888) 208 -> 236, 124 -> 121; 41,389 x
+  // 512 374 -> 442, 203 -> 228; 41,389 x 128 (7760) 118 -> 115, 71 -> 62.
+  // DGBGK_MOM_SPLIT asks for k_moments.
+  if (!std::getenv("DGBGK_MOM_SPLIT") && c.p.V <= 16 * kMomHold) {
+    const int S = c.p.V <= 4 * kMomHold ? 4 : (c.p.V <= 8 * kMomHold ? 8 : 16);
+    const size_t waves = (3 * (size_t)c.p.E + 63) / 64 * S;
+    if (waves <= (c.prec ? 16384 : 8192)) {
+      c.mom_once = 1;
+      c.mom_split = S;
+      c.fuse_mom = 0;
+    }
+  }
   if (const char* fd = std::getenv("DGBGK_FP32_DITHER")) c.dither = fd[0] != '0';
   const Prep& p = c.p;
   // error path of create: release what was made, report the first error
@@ -2244,18 +2395,19 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   }
   const int wall_per = c.wall_ring ? 256 / p.T : 256;  // groups per block
   c.nblk_wall = nwe ? (nwe * c.ngroups + wall_per - 1) / wall_per : 0;
-  // k_moments: one wavefront per 64 nodes leaves fewer than ~8 per SIMD
+  // k_moments (k_moments_once keeps its own split): one wavefront per 64
+  // nodes leaves fewer than ~8 per SIMD
   // below 512k nodes, and then up to four share each node's ordinates.  The
   // choice depends on the node count only, so a mesh gives the same sums
   // (and results) on any device.
   {
     const size_t n3 = 3 * (size_t)p.E;
-    c.mom_split = n3 < (size_t)1 << 19 ? 4 : (n3 < (size_t)1 << 20 ? 2 : 1);
+    if (!c.mom_once) c.mom_split = n3 < (size_t)1 << 19 ? 4 : (n3 < (size_t)1 << 20 ? 2 : 1);
     if (const char* ms = std::getenv("DGBGK_MOM_SPLIT")) {
       const int v = std::atoi(ms);
       if (v == 1 || v == 2 || v == 4) c.mom_split = v;
     }
-    const size_t per = 256 / c.mom_split;
+    const size_t per = c.mom_once ? 64 : 256 / c.mom_split;
     c.nblk_mom = (int)((n3 + per - 1) / per);
   }
   c.neta = (int)p.eta_side.size();
