@@ -2,15 +2,16 @@
 //
 // One step (src/advnce.f90:220-449) is a fixed sequence of launches on the
 // context's stream, with no host synchronisation:
-//   k_eta      FLUCON2 wall mass-flux parameter per type-4 side
 //   k_update   all ordinates of all elements: GTEQNF + GETELC + EDGFLXOPT +
-//              GETINC + ADTHEM + INFLOW, element tiles staged in LDS
+//              GETINC + ADTHEM + INFLOW, element tiles staged in LDS; its
+//              leading blocks FLUCON2's wall mass-flux parameter per type-4 side
 //   k_wall or  in-place sweep order: reflected wall fluxes, every ordinate once
 //   k_wall_ring  what its reflections read is advanced
 //   k_moments or MACROS + COMPMU on f^{k+1}: FP64 sums
-//   k_moments_once
+//   k_moments_once  compensated in FP32
 //   k_points   point averages (GETMAC) when the reference gathers them
-//   k_final    residual max, mass, forces, next DTE (ALOTIM2)
+//   k_final    residual max, mass, forces, next DTE (ALOTIM2); with
+//              k_moments_once by that launch's last block
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -460,6 +461,30 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
   }
 }
 
+// FLUCON2 (src/flucon2.f90:133-233) of type-4 wall side j by the first 256
+// threads of one of the update launch's leading blocks: the wall pass that
+// follows needs it, the update does not, and a launch of its own took 5 us
+// of a 54 us step at 5,763 triangles x 128.
+template <typename T>
+__device__ __forceinline__ void wall_eta(const UpdArgs<T>& a, int j, double* sh) {
+  const int b = a.eta_side[4 * j], e = a.eta_side[4 * j + 1];
+  const int in1 = a.eta_side[4 * j + 2], in2 = a.eta_side[4 * j + 3];
+  const double anx = a.eta_geo[3 * j], any = a.eta_geo[3 * j + 1];
+  const int V = a.V;
+  double s = 0.0;
+  if (threadIdx.x < 256)
+    for (int v = threadIdx.x; v < V; v += 256) {
+      const double test = a.vtd[2 * V + v] * anx + a.vtd[3 * V + v] * any;
+      if (test > 0.0) {
+        const T* fp = a.fcur + (size_t)v * a.ldf + 3 * (size_t)e;
+        const double nf = 0.5 * ((double)fp[in1] + (double)fp[in2]);
+        s += fabs(test) * nf * a.vtd[4 * V + v];
+      }
+    }
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) a.eta[b] = s / a.eta_geo[3 * j + 2];
+}
+
 // kDepth: ordinates whose f is in flight ahead of the one being computed.
 // kDepth + 1 register slots are indexed by compile-time positions of an
 // unrolled loop, so no register copy ever waits on a load still in flight.
@@ -490,7 +515,11 @@ k_update(UpdArgs<T> a) {
   if (sizeof(T) == 4 && threadIdx.x < 4 * kQ)  // read after the first barrier
     s_f[threadIdx.x / 4][kS * 4 + threadIdx.x % 4] = T(0);
   __shared__ double s_red[8];
-  const int logical = xcd_logical(blockIdx.x, gridDim.x);
+  if ((int)blockIdx.x < a.neta) {
+    wall_eta(a, blockIdx.x, s_red);
+    return;
+  }
+  const int logical = xcd_logical(blockIdx.x - a.neta, gridDim.x - a.neta);
   const int tile = logical % a.ntiles;
   const int v0 = (logical / a.ntiles) * a.vchunk;
   const int v1 = min(a.V, v0 + a.vchunk);
@@ -876,6 +905,187 @@ __global__ void __launch_bounds__(256) k_wall_ring(WallArgs<T> a) {
   if (threadIdx.x == 0) a.res_part[a.res_stride + blockIdx.x] = rc;
 }
 
+// Loads and stores past this XCD's caches, for values that blocks of one
+// launch on different XCDs exchange.
+__device__ __forceinline__ double agent_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(double* p, double x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// GETMAC runs on every 1000th step (src/advnce.f90:403-406).
+__device__ __forceinline__ bool gather_step(double steps_done) {
+  return ((long long)steps_done + 1) % 1000 == 0;
+}
+
+// MACROS point averages (src/macros.f90:156-188) of point q over the point
+// CSR; gather: also GETMAC's copy of the pressure for GETFOR.
+__device__ __forceinline__ void point_average(int q, const double* __restrict__ mom,
+                                              const double* __restrict__ rj,
+                                              const int* __restrict__ ptr,
+                                              const int* __restrict__ node,
+                                              double* __restrict__ pts,
+                                              double* __restrict__ ps_glob, int E, int P,
+                                              double mm, double rgas, int gather) {
+  const size_t N3 = 3 * (size_t)E;
+  double flag = 0, nd = 0, u = 0, vv = 0, ps = 0;
+  for (int i = ptr[q]; i < ptr[q + 1]; ++i) {
+    const int k = node[i];
+    const double ae = rj[k / 3];
+    const double n = mom[k];
+    if (n >= 1e-20) {
+      u += ae * mom[N3 + k];
+      vv += ae * mom[2 * N3 + k];
+    }
+    flag += ae;
+    nd += n * ae;
+    ps += mom[3 * N3 + k] * ae;
+  }
+  double rho = 0, t = 0;
+  if (nd < 1e-20) {
+    u = vv = ps = 0.0;
+  } else {
+    nd = nd / flag;
+    rho = nd * mm;
+    u = u / flag;
+    vv = vv / flag;
+    ps = ps / flag;
+    t = ps / (rgas * rho);
+  }
+  pts[q] = nd;
+  pts[P + q] = rho;
+  pts[2 * P + q] = u;
+  pts[3 * P + q] = vv;
+  pts[4 * P + q] = ps;
+  pts[5 * P + q] = t;
+  if (gather) ps_glob[q] = ps;
+}
+
+// Step epilogue: GETRES max, mass, GETFOR (src/getfor.f90:29-49) on the
+// gathered point pressure, the residual record, and ALOTIM2's next DTE, by
+// one block of at most 1024 threads.
+__device__ __forceinline__ void final_body(const FinalArgs& a, double (&s_red)[6][16]) {
+  double* const scal = a.scal;
+  const double steps_done = scal[6];  // in flight with the partials below
+  double r = 0.0, rc = 0.0, m = 0.0, ms = 0.0, lift = 0.0, drag = 0.0;
+  // each thread's partials, up to kLd per array loaded before any is
+  // combined (one memory latency instead of one per partial); combined in
+  // index order, so the mass sum keeps its order (out-of-range slots add
+  // 0 and all partials are >= 0)
+  constexpr int kLd = 8;
+  const int nt = blockDim.x, nres = a.nres, nmom = a.nmom;
+  for (int b = threadIdx.x; b < nres; b += kLd * nt) {
+    double x[kLd], y[kLd];
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      const int i = b + j * nt;
+      x[j] = i < nres ? a.res_part[i] : 0.0;
+      y[j] = i < nres ? a.res_part[nres + i] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      r = fmax(r, x[j]);
+      rc = fmax(rc, y[j]);
+    }
+  }
+  // (agent scope: the moments launch that ends with this may have written
+  // them from other XCDs)
+  for (int b = threadIdx.x; b < nmom; b += kLd * nt) {
+    double x[kLd], y[kLd];
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      const int i = b + j * nt;
+      x[j] = i < nmom ? agent_load(a.mu_part + i) : 0.0;
+      y[j] = i < nmom ? agent_load(a.mass_part + i) : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      m = fmax(m, x[j]);
+      ms += y[j];
+    }
+  }
+  // In a step, GETMAC on every 1000th step (src/advnce.f90:403-406): the
+  // point averages and the gathered pressure that GETFOR below uses.  Rare,
+  // so this block does it rather than a launch every step.
+  if (a.record >= 0 && gather_step(steps_done)) {
+    for (int q = threadIdx.x; q < a.P; q += blockDim.x)
+      point_average(q, a.mom, a.rj, a.ptr, a.node, a.pts, a.ps_glob, a.E, a.P, a.mm, a.rgas, 1);
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < a.nf; i += blockDim.x) {
+    const int p1 = a.fside[2 * i], p2 = a.fside[2 * i + 1];
+    const double x1 = a.coord[2 * p1], y1 = a.coord[2 * p1 + 1];
+    const double x2 = a.coord[2 * p2], y2 = a.coord[2 * p2 + 1];
+    const double len = sqrt((x2 - x1) * (x2 - x1) + (y2 - y1) * (y2 - y1));
+    const double px = -(y2 - y1), py = x2 - x1;
+    const double mag = sqrt(px * px + py * py);
+    const double psav = 0.5 * (a.ps_glob[p1] + a.ps_glob[p2]);
+    lift -= psav * len * (py / mag);
+    drag -= psav * len * (px / mag);
+  }
+  // the three maxima and three sums in one LDS round: each wavefront
+  // reduces its six values, then thread j combines value j over the
+  // wavefronts in wavefront order (the order of block_max / block_sum)
+  for (int o = 32; o > 0; o >>= 1) {
+    r = fmax(r, __shfl_down(r, o, 64));
+    rc = fmax(rc, __shfl_down(rc, o, 64));
+    m = fmax(m, __shfl_down(m, o, 64));
+    ms += __shfl_down(ms, o, 64);
+    lift += __shfl_down(lift, o, 64);
+    drag += __shfl_down(drag, o, 64);
+  }
+  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    s_red[0][w] = r;
+    s_red[1][w] = rc;
+    s_red[2][w] = m;
+    s_red[3][w] = ms;
+    s_red[4][w] = lift;
+    s_red[5][w] = drag;
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int j = threadIdx.x;
+    double x = s_red[j][0];
+    for (int i = 1; i < nw; ++i) x = j < 3 ? fmax(x, s_red[j][i]) : x + s_red[j][i];
+    s_red[j][0] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    r = s_red[0][0];
+    rc = s_red[1][0];
+    m = s_red[2][0];
+    ms = s_red[3][0];
+    lift = s_red[4][0];
+    drag = s_red[5][0];
+    if (a.record >= 0) {
+      // scal[6] counts completed steps (ITIME of src/advnce.f90:220)
+      const long long itime = (long long)scal[6] + 1;
+      scal[6] = (double)itime;
+      const int slot = (int)((itime - 1) % a.rec_cap);
+      if (itime == 1) scal[1] = r;
+      a.rec[slot].sumres = r;
+      a.rec[slot].logres = log(r / scal[1]);
+      a.rec[slot].dte = scal[0];
+      a.rec[slot].mass = ms;
+      a.rec[slot].lift = lift;
+      a.rec[slot].drag = drag;
+      a.rec[slot].change = rc;
+    }
+    scal[2] = lift;
+    scal[3] = drag;
+    scal[5] = ms;
+    const double dteb = (m > 0.0) ? 0.9 * (1 / m) : 1000000.0;
+    scal[0] = dteb < scal[4] ? dteb : scal[4];
+  }
+}
+
+__global__ void __launch_bounds__(1024) k_final(FinalArgs a) {
+  __shared__ double s_red[6][16];
+  final_body(a, s_red);
+}
+
 // ---------------------------------------------------------------------------
 // k_moments: MACROS (src/macros.f90:80-164) and COMPMU
 // (src/compmu.f90:36-97) per DG node, FP64 compensated sums over all ordinates.  Pass 1:
@@ -1149,6 +1359,8 @@ template <typename T, int S>
 __global__ void __launch_bounds__(64 * S) k_moments_once(MomArgs<T> a) {
   constexpr bool kComp = sizeof(T) < sizeof(double);
   __shared__ double s_part[S][3][64];
+  __shared__ double s_red[6][16];
+  __shared__ int s_last;
   const int lane = threadIdx.x & 63;
   const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t N3 = 3 * (size_t)a.E, k = (size_t)blockIdx.x * 64 + lane;
@@ -1238,86 +1450,36 @@ __global__ void __launch_bounds__(64 * S) k_moments_once(MomArgs<T> a) {
     }
     node_result(a, k, n, ux, uy, tp - ep, tt - et, mu, mass);
   }
-  // only the first wavefront holds results
+  // Only the first wavefront holds results.  In a step the block that is
+  // last to leave its partials runs the epilogue (its own launch took 6 us
+  // of a 54 us step at 5,763 triangles x 128): each block's are past the
+  // caches before it counts itself, and on GETMAC's steps, where the epilogue
+  // reads every node field, those are too.
+  const bool last = a.fin.record >= 0;
+  const bool gather = last && gather_step(a.fin.scal[6]);
   if (sub == 0) {
     for (int o = 32; o > 0; o >>= 1) {
       mu = fmax(mu, __shfl_down(mu, o, 64));
       mass += __shfl_down(mass, o, 64);
     }
     if (lane == 0) {
-      a.mu_part[blockIdx.x] = mu;
-      a.mass_part[blockIdx.x] = mass;
+      agent_store(a.mu_part + blockIdx.x, mu);
+      agent_store(a.mass_part + blockIdx.x, mass);
+    }
+    if (last) {
+      if (gather) __threadfence();
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0)
+        s_last = __hip_atomic_fetch_add(a.fin.count, 1, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
     }
   }
-}
-
-// FLUCON2 (src/flucon2.f90:133-233): one block per type-4 wall side.
-template <typename T>
-__global__ void __launch_bounds__(256) k_eta(const T* __restrict__ f,
-                                             const int* __restrict__ side,
-                                             const double* __restrict__ geo,
-                                             const double* __restrict__ vtd,
-                                             double* __restrict__ eta, int E, int V,
-                                             long long ldf) {
-  __shared__ double s_red[8];
-  const int j = blockIdx.x;
-  const int b = side[4 * j], e = side[4 * j + 1], in1 = side[4 * j + 2], in2 = side[4 * j + 3];
-  const double anx = geo[3 * j], any = geo[3 * j + 1], bottom = geo[3 * j + 2];
-  const size_t N3 = 3 * (size_t)E;
-  double s = 0.0;
-  for (int v = threadIdx.x; v < V; v += blockDim.x) {
-    const double test = vtd[2 * V + v] * anx + vtd[3 * V + v] * any;
-    if (test > 0.0) {
-      const T* fp = f + (size_t)v * ldf + 3 * (size_t)e;
-      const double nf = 0.5 * ((double)fp[in1] + (double)fp[in2]);
-      s += fabs(test) * nf * vtd[4 * V + v];
-    }
-  }
-  s = block_sum(s, s_red);
-  if (threadIdx.x == 0) eta[b] = s / bottom;
-}
-
-// MACROS point averages (src/macros.f90:156-188) of point q over the point
-// CSR; gather: also GETMAC's copy of the pressure for GETFOR.
-__device__ __forceinline__ void point_average(int q, const double* __restrict__ mom,
-                                              const double* __restrict__ rj,
-                                              const int* __restrict__ ptr,
-                                              const int* __restrict__ node,
-                                              double* __restrict__ pts,
-                                              double* __restrict__ ps_glob, int E, int P,
-                                              double mm, double rgas, int gather) {
-  const size_t N3 = 3 * (size_t)E;
-  double flag = 0, nd = 0, u = 0, vv = 0, ps = 0;
-  for (int i = ptr[q]; i < ptr[q + 1]; ++i) {
-    const int k = node[i];
-    const double ae = rj[k / 3];
-    const double n = mom[k];
-    if (n >= 1e-20) {
-      u += ae * mom[N3 + k];
-      vv += ae * mom[2 * N3 + k];
-    }
-    flag += ae;
-    nd += n * ae;
-    ps += mom[3 * N3 + k] * ae;
-  }
-  double rho = 0, t = 0;
-  if (nd < 1e-20) {
-    u = vv = ps = 0.0;
-  } else {
-    nd = nd / flag;
-    rho = nd * mm;
-    u = u / flag;
-    vv = vv / flag;
-    ps = ps / flag;
-    t = ps / (rgas * rho);
-  }
-  pts[q] = nd;
-  pts[P + q] = rho;
-  pts[2 * P + q] = u;
-  pts[3 * P + q] = vv;
-  pts[4 * P + q] = ps;
-  pts[5 * P + q] = t;
-  if (gather) ps_glob[q] = ps;
+  if (!last) return;
+  __syncthreads();
+  if (!s_last) return;
+  if (gather) __threadfence();
+  final_body(a.fin, s_red);
+  if (threadIdx.x == 0) *a.fin.count = 0;  // for the next launch
 }
 
 __global__ void __launch_bounds__(256) k_points(const double* __restrict__ mom,
@@ -1329,141 +1491,6 @@ __global__ void __launch_bounds__(256) k_points(const double* __restrict__ mom,
                                                 int P, double mm, double rgas, int gather) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q < P) point_average(q, mom, rj, ptr, node, pts, ps_glob, E, P, mm, rgas, gather);
-}
-
-struct PointArgs {
-  const double* mom;
-  const double* rj;
-  const int* ptr;
-  const int* node;
-  double* pts;
-  int E, P;
-  double mm, rgas;
-};
-
-// Step epilogue: GETRES max, mass, GETFOR (src/getfor.f90:29-49) on the
-// gathered point pressure, the residual record, and ALOTIM2's next DTE.
-__global__ void __launch_bounds__(1024) k_final(const double* __restrict__ res_part, int nres,
-                                               const double* __restrict__ mu_part,
-                                               const double* __restrict__ mass_part, int nmom,
-                                               const int* __restrict__ fside, int nf,
-                                               const double* __restrict__ coord,
-                                               double* __restrict__ ps_glob,
-                                               double* __restrict__ scal,
-                                               StepRec* __restrict__ rec, int rec_cap,
-                                               int record, PointArgs pa) {
-  __shared__ double s_red[6][16];
-  const double steps_done = scal[6];  // in flight with the partials below
-  double r = 0.0, rc = 0.0, m = 0.0, ms = 0.0, lift = 0.0, drag = 0.0;
-  // each thread's partials, up to kLd per array loaded before any is
-  // combined (one memory latency instead of one per partial); combined in
-  // index order, so the mass sum keeps its order (out-of-range slots add
-  // 0 and all partials are >= 0)
-  constexpr int kLd = 8;
-  const int nt = blockDim.x;
-  for (int b = threadIdx.x; b < nres; b += kLd * nt) {
-    double x[kLd], y[kLd];
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      const int i = b + j * nt;
-      x[j] = i < nres ? res_part[i] : 0.0;
-      y[j] = i < nres ? res_part[nres + i] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      r = fmax(r, x[j]);
-      rc = fmax(rc, y[j]);
-    }
-  }
-  for (int b = threadIdx.x; b < nmom; b += kLd * nt) {
-    double x[kLd], y[kLd];
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      const int i = b + j * nt;
-      x[j] = i < nmom ? mu_part[i] : 0.0;
-      y[j] = i < nmom ? mass_part[i] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      m = fmax(m, x[j]);
-      ms += y[j];
-    }
-  }
-  // In a step, GETMAC on every 1000th step (src/advnce.f90:403-406): the
-  // point averages and the gathered pressure that GETFOR below uses.  Rare,
-  // so this block does it rather than a launch every step.
-  if (record >= 0 && (((long long)steps_done + 1) % 1000) == 0) {
-    for (int q = threadIdx.x; q < pa.P; q += blockDim.x)
-      point_average(q, pa.mom, pa.rj, pa.ptr, pa.node, pa.pts, ps_glob, pa.E, pa.P, pa.mm,
-                    pa.rgas, 1);
-    __syncthreads();
-  }
-  for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-    const int p1 = fside[2 * i], p2 = fside[2 * i + 1];
-    const double x1 = coord[2 * p1], y1 = coord[2 * p1 + 1];
-    const double x2 = coord[2 * p2], y2 = coord[2 * p2 + 1];
-    const double len = sqrt((x2 - x1) * (x2 - x1) + (y2 - y1) * (y2 - y1));
-    const double px = -(y2 - y1), py = x2 - x1;
-    const double mag = sqrt(px * px + py * py);
-    const double psav = 0.5 * (ps_glob[p1] + ps_glob[p2]);
-    lift -= psav * len * (py / mag);
-    drag -= psav * len * (px / mag);
-  }
-  // the three maxima and three sums in one LDS round: each wavefront
-  // reduces its six values, then thread j combines value j over the
-  // wavefronts in wavefront order (the order of block_max / block_sum)
-  for (int o = 32; o > 0; o >>= 1) {
-    r = fmax(r, __shfl_down(r, o, 64));
-    rc = fmax(rc, __shfl_down(rc, o, 64));
-    m = fmax(m, __shfl_down(m, o, 64));
-    ms += __shfl_down(ms, o, 64);
-    lift += __shfl_down(lift, o, 64);
-    drag += __shfl_down(drag, o, 64);
-  }
-  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    s_red[0][w] = r;
-    s_red[1][w] = rc;
-    s_red[2][w] = m;
-    s_red[3][w] = ms;
-    s_red[4][w] = lift;
-    s_red[5][w] = drag;
-  }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int j = threadIdx.x;
-    double x = s_red[j][0];
-    for (int i = 1; i < nw; ++i) x = j < 3 ? fmax(x, s_red[j][i]) : x + s_red[j][i];
-    s_red[j][0] = x;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    r = s_red[0][0];
-    rc = s_red[1][0];
-    m = s_red[2][0];
-    ms = s_red[3][0];
-    lift = s_red[4][0];
-    drag = s_red[5][0];
-    if (record >= 0) {
-      // scal[6] counts completed steps (ITIME of src/advnce.f90:220)
-      const long long itime = (long long)scal[6] + 1;
-      scal[6] = (double)itime;
-      const int slot = (int)((itime - 1) % rec_cap);
-      if (itime == 1) scal[1] = r;
-      rec[slot].sumres = r;
-      rec[slot].logres = log(r / scal[1]);
-      rec[slot].dte = scal[0];
-      rec[slot].mass = ms;
-      rec[slot].lift = lift;
-      rec[slot].drag = drag;
-      rec[slot].change = rc;
-    }
-    scal[2] = lift;
-    scal[3] = drag;
-    scal[5] = ms;
-    const double dteb = (m > 0.0) ? 0.9 * (1 / m) : 1000000.0;
-    scal[0] = dteb < scal[4] ? dteb : scal[4];
-  }
 }
 
 // Maxwellian seed per DG node from per-point (n, beta^2, u, v): the INICON2
@@ -1646,6 +1673,7 @@ struct Ctx {
          *pts = nullptr, *ps_glob = nullptr, *coord = nullptr, *res_part = nullptr,
          *mu_part = nullptr, *mass_part = nullptr, *scal = nullptr, *ps4 = nullptr,
          *msum = nullptr;
+  int* count = nullptr;     // moments blocks done in this launch
   float* ephase = nullptr;  // [E] FP32 store dither phase per element
   StepRec* rec = nullptr;
   int rec_cap = 0;
@@ -1675,9 +1703,22 @@ struct Ctx {
 
 namespace {
 
-// partials: k_update of this step left the first moment pass in msum
+FinalArgs final_args(const Ctx& c, int record) {
+  FinalArgs a;
+  a.res_part = c.res_part; a.nres = c.nblk_upd + c.nblk_wall;
+  a.mu_part = c.mu_part; a.mass_part = c.mass_part; a.nmom = c.nblk_mom;
+  a.fside = c.fside; a.nf = c.nforce; a.coord = c.coord; a.ps_glob = c.ps_glob;
+  a.scal = c.scal; a.rec = c.rec; a.rec_cap = c.rec_cap; a.record = record;
+  a.mom = c.mom; a.rj = c.rj; a.ptr = c.pt_ptr; a.node = c.pt_node; a.pts = c.pts;
+  a.E = c.p.E; a.P = c.p.P; a.mm = c.p.prm.m / kNa; a.rgas = c.p.prm.rgas;
+  a.count = c.count;
+  return a;
+}
+
+// in_step: after k_update and the wall pass, whose sums (if it leaves any)
+// are in msum; k_moments_once then also runs the step's epilogue
 template <typename T>
-int launch_moments(Ctx& c, bool partials = false) {
+int launch_moments(Ctx& c, bool in_step = false) {
   MomArgs<T> m;
   m.f = (const T*)c.f[c.cur];
   m.vtd = c.vtd;
@@ -1689,35 +1730,33 @@ int launch_moments(Ctx& c, bool partials = false) {
   m.mass_part = c.mass_part;
   m.mm = c.p.prm.m / kNa;
   m.sigt = kPi * c.p.prm.d * c.p.prm.d;
-  m.msum = partials ? c.msum : nullptr;
+  m.msum = in_step && c.fuse_mom ? c.msum : nullptr;
   m.ewslot = c.ewslot;
   m.nchunks = c.nvchunks;
   m.vchunk = c.vchunk;
   m.E = c.p.E;
   m.ldf = (long long)c.ldf;
   m.V = c.p.V;
+  m.fin = final_args(c, c.mom_once && in_step ? 0 : -1);
+  const dim3 g(c.nblk_mom);
   if (c.mom_once && c.mom_split == 4)
-    hipLaunchKernelGGL((k_moments_once<T, 4>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments_once<T, 4>), g, dim3(256), 0, c.stream, m);
   else if (c.mom_once && c.mom_split == 8)
-    hipLaunchKernelGGL((k_moments_once<T, 8>), dim3(c.nblk_mom), dim3(512), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments_once<T, 8>), g, dim3(512), 0, c.stream, m);
   else if (c.mom_once)
-    hipLaunchKernelGGL((k_moments_once<T, 16>), dim3(c.nblk_mom), dim3(1024), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments_once<T, 16>), g, dim3(1024), 0, c.stream, m);
   else if (c.mom_split == 4)
-    hipLaunchKernelGGL((k_moments<T, 4>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments<T, 4>), g, dim3(256), 0, c.stream, m);
   else if (c.mom_split == 2)
-    hipLaunchKernelGGL((k_moments<T, 2>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments<T, 2>), g, dim3(256), 0, c.stream, m);
   else
-    hipLaunchKernelGGL((k_moments<T, 1>), dim3(c.nblk_mom), dim3(256), 0, c.stream, m);
+    hipLaunchKernelGGL((k_moments<T, 1>), g, dim3(256), 0, c.stream, m);
   HIPCK(hipGetLastError());
   return kOk;
 }
 
 int launch_final(Ctx& c, int record) {
-  PointArgs pa{c.mom, c.rj, c.pt_ptr, c.pt_node, c.pts, c.p.E, c.p.P, c.p.prm.m / kNa,
-               c.p.prm.rgas};
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(1024), 0, c.stream, c.res_part,
-                     c.nblk_upd + c.nblk_wall, c.mu_part, c.mass_part, c.nblk_mom, c.fside,
-                     c.nforce, c.coord, c.ps_glob, c.scal, c.rec, c.rec_cap, record, pa);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(1024), 0, c.stream, final_args(c, record));
   HIPCK(hipGetLastError());
   return kOk;
 }
@@ -1769,7 +1808,7 @@ void tend(Ctx& c, int k) {
 
 template <typename T, int kS>
 void launch_update_s(Ctx& c, const UpdArgs<T>& u) {
-  const dim3 g(c.nblk_upd), b(kS);
+  const dim3 g(c.neta + c.nblk_upd), b(kS);
   if (u.cmminc) {  // IMMAT = 0 runs at prefetch depth 1 (set at create)
     if (c.fuse_mom)
       hipLaunchKernelGGL((k_update<T, 1, true, kS, true>), g, b, 0, c.stream, u);
@@ -1829,18 +1868,12 @@ int step_once(Ctx& c) {
   const Prep& p = c.p;
   const T* fc = (const T*)c.f[c.cur];
   T* fn = (T*)c.f[1 - c.cur];
-  if (c.neta) {
-    tbegin(c, 3);
-    hipLaunchKernelGGL(k_eta<T>, dim3(c.neta), dim3(256), 0, c.stream, fc, c.eta_side,
-                       c.eta_geo, c.vtd, c.eta, p.E, p.V, (long long)c.ldf);
-    HIPCK(hipGetLastError());
-    tend(c, 3);
-  }
   UpdArgs<T> u;
   u.fcur = fc; u.fnxt = fn; u.geo = (const T*)c.geo; u.uinfo = c.uinfo;
   u.unx = (const T*)c.unx; u.uny = (const T*)c.uny;
   u.emask = c.emask; u.ewslot = c.ewslot; u.np = (const T*)c.np; u.vrow = (const T*)c.vrow;
   u.tiles = c.tiles; u.halo = c.halo; u.wpart = (T*)c.wpart; u.msum = c.msum;
+  u.vtd = c.vtd; u.eta_side = c.eta_side; u.eta_geo = c.eta_geo; u.eta = c.eta; u.neta = c.neta;
   u.scal = c.scal; u.res_part = c.res_part; u.res_stride = c.nblk_upd + c.nblk_wall;
   u.E = p.E; u.V = p.V; u.ntiles = c.ntiles; u.vchunk = c.vchunk;
   u.ephase = c.ephase;
@@ -1877,9 +1910,10 @@ int step_once(Ctx& c) {
   }
   c.cur = 1 - c.cur;
   tbegin(c, 2);
-  int st = launch_moments<T>(c, c.fuse_mom != 0);
+  int st = launch_moments<T>(c, true);
   if (st) return st;
   tend(c, 2);
+  if (c.mom_once) return kOk;
   tbegin(c, 4);
   st = launch_final(c, 0);  // with GETMAC's point gather every 1000th step
   tend(c, 4);
@@ -2107,6 +2141,7 @@ int upload_tables(Ctx& c) {
   if ((st = upload(&c.intma, p.intma, c.owned))) return st;
   std::vector<double> eta0(std::max(p.B, 1), 0.0);
   if ((st = upload(&c.eta, eta0, c.owned))) return st;
+  if ((st = upload(&c.count, std::vector<int>{0}, c.owned))) return st;
   if ((st = alloc((T**)&c.np, 5 * N3, c.owned))) return st;
   if ((st = alloc(&c.mom, 5 * N3, c.owned))) return st;
   if ((st = alloc(&c.pts, 6 * (size_t)p.P, c.owned))) return st;

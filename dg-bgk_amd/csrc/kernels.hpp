@@ -66,6 +66,11 @@ struct UpdArgs {
   const double* __restrict__ scal; // [0] = DTE
   double* __restrict__ res_part;   // per block: max|increment|; +res_stride: max|change|
   const float* __restrict__ ephase; // [E] FP32 store dither phase per element
+  const double* __restrict__ vtd;  // [8][V] and the FLUCON2 sides of the leading blocks:
+  const int* __restrict__ eta_side;    // [neta][4] side, element, its two nodes
+  const double* __restrict__ eta_geo;  // [neta][3] normal, denominator
+  double* __restrict__ eta;
+  int neta;
   int res_stride;
   int E, V, ntiles, vchunk;
   long long ldf;  // row stride of f
@@ -104,6 +109,28 @@ struct WallArgs {
   int cmminc;     // IMMAT = 0: as in UpdArgs
 };
 
+// The step's epilogue (k_final).
+struct FinalArgs {
+  const double* res_part;  // [2][nres] of the update and wall passes
+  const double* mu_part;   // [nmom] of the moments blocks
+  const double* mass_part;
+  const int* fside;        // [nf][2] points of the force sides
+  const double* coord;
+  double* ps_glob;
+  double* scal;
+  StepRec* rec;
+  const double* mom;       // GETMAC's point gather, on every 1000th step
+  const double* rj;
+  const int* ptr;
+  const int* node;
+  double* pts;
+  int* count;              // moments blocks done (k_moments_once)
+  int nres, nmom, nf, rec_cap;
+  int record;              // < 0: outside a step
+  int E, P;
+  double mm, rgas;
+};
+
 template <typename T>
 struct MomArgs {
   const T* __restrict__ f;
@@ -120,6 +147,7 @@ struct MomArgs {
   double mm, sigt;
   int E, V, nchunks, vchunk;
   long long ldf;  // row stride of f
+  FinalArgs fin;  // k_moments_once; record < 0: no epilogue
 };
 
 }  // namespace dgbgk
