@@ -1494,23 +1494,45 @@ __global__ void __launch_bounds__(256) k_points(const double* __restrict__ mom,
 }
 
 // Maxwellian seed per DG node from per-point (n, beta^2, u, v): the INICON2
-// formula (src/inicon2.f90:149-163) with point-wise state.
-template <typename T>
+// formula (src/inicon2.f90:149-163) with point-wise state.  A thread keeps
+// its node's state over a chunk of ordinates (blockIdx.y), whose scalars are
+// scalar loads, and stores past the L2; bound by writing f.  With one thread
+// per value, which gathered the state again for each, 1,005,669 x 2048 took
+// 29 ms (FP64) and 26 ms (FP32); so it takes 10.5 (4.7 TB/s) and 8.8, the
+// latter bound by the exponential.
+// kMom: also leaves the chunk's first-pass moment sums, as k_update does, so
+// the moments launch that follows reads f once.
+template <typename T, bool kMom>
 __global__ void __launch_bounds__(256) k_seed(T* __restrict__ f, const int* __restrict__ intma,
                                               const double* __restrict__ ps4,
-                                              const double* __restrict__ vtd, int E, int V,
+                                              const double* __restrict__ vtd,
+                                              double* __restrict__ msum, int vchunk, int E, int V,
                                               int P, long long ldf) {
   const size_t N3 = 3 * (size_t)E;
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int v = blockIdx.y;
   if (k >= N3) return;
   const int q = intma[k] - 1;
   const double n1 = ps4[q], b2 = ps4[P + q], u0 = ps4[2 * P + q], v0 = ps4[3 * P + q];
-  const double ux = vtd[2 * V + v], uy = vtd[3 * V + v];
-  const double tmp = (ux - u0) * (ux - u0) + (uy - v0) * (uy - v0);
-  const double sp = sqrt(tmp);
-  const double f0 = (b2 / 3.1416) * exp(-(b2 * (sp * sp)));
-  f[(size_t)v * ldf + k] = (T)(n1 * f0);
+  const double c0 = b2 / 3.1416;
+  const int vb = blockIdx.y * vchunk, ve = min(V, vb + vchunk);
+  double m0 = 0.0, m1 = 0.0, m2 = 0.0;
+  T* o = f + (size_t)vb * ldf + k;
+  for (int v = vb; v < ve; ++v, o += ldf) {
+    const double dx = ldc(vtd, 2 * V + v) - u0, dy = ldc(vtd, 3 * V + v) - v0;
+    const T x = (T)(n1 * (c0 * mexp(-(b2 * (dx * dx + dy * dy)))));
+    fstore_nt(o, x);
+    if (kMom) {
+      m0 = fma(ldc(vtd, 4 * V + v), (double)x, m0);
+      m1 = fma(ldc(vtd, 5 * V + v), (double)x, m1);
+      m2 = fma(ldc(vtd, 6 * V + v), (double)x, m2);
+    }
+  }
+  if (kMom) {
+    double* ms = msum + (size_t)blockIdx.y * 3 * N3 + k;
+    ms[0] = m0;
+    ms[N3] = m1;
+    ms[2 * N3] = m2;
+  }
 }
 
 // Minimum, maximum and count of non-finite values of f, per block: rows v
@@ -1715,10 +1737,11 @@ FinalArgs final_args(const Ctx& c, int record) {
   return a;
 }
 
-// in_step: after k_update and the wall pass, whose sums (if it leaves any)
-// are in msum; k_moments_once then also runs the step's epilogue
+// sums: the kernel that wrote f left its first-pass sums in msum (if it
+// leaves any: fuse_mom); in_step: k_moments_once also runs the step's
+// epilogue
 template <typename T>
-int launch_moments(Ctx& c, bool in_step = false) {
+int launch_moments(Ctx& c, bool sums, bool in_step) {
   MomArgs<T> m;
   m.f = (const T*)c.f[c.cur];
   m.vtd = c.vtd;
@@ -1730,7 +1753,7 @@ int launch_moments(Ctx& c, bool in_step = false) {
   m.mass_part = c.mass_part;
   m.mm = c.p.prm.m / kNa;
   m.sigt = kPi * c.p.prm.d * c.p.prm.d;
-  m.msum = in_step && c.fuse_mom ? c.msum : nullptr;
+  m.msum = sums && c.fuse_mom ? c.msum : nullptr;
   m.ewslot = c.ewslot;
   m.nchunks = c.nvchunks;
   m.vchunk = c.vchunk;
@@ -1910,7 +1933,7 @@ int step_once(Ctx& c) {
   }
   c.cur = 1 - c.cur;
   tbegin(c, 2);
-  int st = launch_moments<T>(c, true);
+  int st = launch_moments<T>(c, true, true);
   if (st) return st;
   tend(c, 2);
   if (c.mom_once) return kOk;
@@ -2163,17 +2186,22 @@ int seed_points(Ctx& c, const std::vector<double>& ps4) {
   HIPCK(hipMemcpyAsync(c.ps4, ps4.data(), ps4.size() * sizeof(double), hipMemcpyHostToDevice,
                        c.stream));
   const size_t N3 = 3 * (size_t)c.p.E;
-  hipLaunchKernelGGL(k_seed<T>, dim3((unsigned)((N3 + 255) / 256), c.p.V), dim3(256), 0,
-                     c.stream, (T*)c.f[c.cur], c.intma, c.ps4, c.vtd, c.p.E, c.p.V, c.p.P,
-                     (long long)c.ldf);
+  const dim3 g((unsigned)((N3 + 255) / 256), c.nvchunks);
+  if (c.fuse_mom)
+    hipLaunchKernelGGL((k_seed<T, true>), g, dim3(256), 0, c.stream, (T*)c.f[c.cur], c.intma,
+                       c.ps4, c.vtd, c.msum, c.vchunk, c.p.E, c.p.V, c.p.P, (long long)c.ldf);
+  else
+    hipLaunchKernelGGL((k_seed<T, false>), g, dim3(256), 0, c.stream, (T*)c.f[c.cur], c.intma,
+                       c.ps4, c.vtd, c.msum, c.vchunk, c.p.E, c.p.V, c.p.P, (long long)c.ldf);
   HIPCK(hipGetLastError());
   return kOk;
 }
 
 // after f changes outside a step: initial MACROS + GETMAC + first DTE
+// (sums: whoever wrote f left its first-pass sums)
 template <typename T>
-int refresh(Ctx& c) {
-  int st = launch_moments<T>(c);
+int refresh(Ctx& c, bool sums) {
+  int st = launch_moments<T>(c, sums, false);
   if (st) return st;
   if ((st = launch_points(c, 1))) return st;
   // DTE for the next step, no record
@@ -2181,7 +2209,9 @@ int refresh(Ctx& c) {
   return launch_final(c, -1);
 }
 
-int do_refresh(Ctx& c) { return c.prec ? refresh<float>(c) : refresh<double>(c); }
+int do_refresh(Ctx& c, bool sums) {
+  return c.prec ? refresh<float>(c, sums) : refresh<double>(c, sums);
+}
 
 }  // namespace
 }  // namespace dgbgk
@@ -2478,7 +2508,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
     st = c.prec ? seed_points<float>(c, ps4) : seed_points<double>(c, ps4);
     if (st) return cleanup(st);
   }
-  if ((st = do_refresh(c))) return cleanup(st);
+  if ((st = do_refresh(c, true))) return cleanup(st);
   if (hipStreamSynchronize(c.stream) != hipSuccess)
     return cleanup(fail(kErrHip, "initialisation failed on the device"));
   *out = h;
@@ -2564,7 +2594,7 @@ int dgbgk_set_f(dgbgk_ctx* h, const double* f) {
     hipLaunchKernelGGL(k_to_device<double>, g, dim3(256), 0, c.stream, d,
                        (double*)c.f[c.cur], (const int*)c.d_eorder, c.p.E, c.p.V,
                        (long long)c.ldf);
-  int st = do_refresh(c);
+  int st = do_refresh(c, false);
   hipError_t e2 = hipStreamSynchronize(c.stream);
   const hipError_t e3 = hipFree(d);
   if (st) return st;
@@ -2589,7 +2619,7 @@ int dgbgk_seed_maxwellian(dgbgk_ctx* h, const double* rho, const double* u, cons
   }
   int st = c.prec ? seed_points<float>(c, ps4) : seed_points<double>(c, ps4);
   if (st) return st;
-  if ((st = do_refresh(c))) return st;
+  if ((st = do_refresh(c, true))) return st;
   HIPCK(hipStreamSynchronize(c.stream));
   return kOk;
 }
