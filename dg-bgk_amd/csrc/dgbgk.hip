@@ -1092,11 +1092,12 @@ __global__ void __launch_bounds__(1024) k_final(FinalArgs a) {
 // n, n*u, n*v; pass 2: pressure and mean relative speed about u.  Writes the
 // FP64 node fields and the next step's GTEQNF/COMPMU parameters in T.
 // ---------------------------------------------------------------------------
-// k_moments geometry: a block of 256 threads serves 256 / S nodes with S
-// wavefronts per node, each summing its share of the ordinates; the shares
-// combine through LDS in wavefront order.  Few nodes give few wavefronts
-// (one per 64 nodes at S = 1), too few to hide FP64 latency; many nodes
-// keep the chip busy at S = 1, where the combine would only cost.
+// k_moments geometry: a block of 256 threads (512 at S = 8) serves 256 / S
+// (64) nodes with S wavefronts per node, each summing its share of the
+// ordinates; the shares combine through LDS in wavefront order.  Few nodes
+// give few wavefronts (one per 64 nodes at S = 1), too few to hide memory
+// and FP64 latency; many nodes keep the chip busy at S = 1, where the combine
+// would only cost.
 // kMomRing: register sets of four ordinates each wavefront keeps in its
 // load ring.
 #ifndef DGBGK_MOM_RING32
@@ -1141,10 +1142,10 @@ __device__ __forceinline__ void node_result(const MomArgs<T>& a, size_t k, doubl
 }
 
 template <typename T, int S>
-__global__ void __launch_bounds__(256) k_moments(MomArgs<T> a) {
+__global__ void __launch_bounds__(S > 4 ? 64 * S : 256) k_moments(MomArgs<T> a) {
   constexpr bool kComp = sizeof(T) < sizeof(double);
-  constexpr int kMomNodes = 256 / S;
-  __shared__ double s_red[8];
+  constexpr int kMomNodes = (S > 4 ? 64 * S : 256) / S;
+  __shared__ double s_red[16];
   __shared__ double s_part[S > 1 ? S : 1][6][S > 1 ? kMomNodes : 1];
   // the wavefront's share index, made a scalar: the ordinate loops then
   // read the velocity tables with scalar loads
@@ -1258,69 +1259,66 @@ __global__ void __launch_bounds__(256) k_moments(MomArgs<T> a) {
       const double dx = ldc(cxb, v) - ux, dy = ldc(cyb, v) - uy;
       const double ex = ux - ldc(cxa, v), ey = uy - ldc(cya, v);
       sp += 0.5 * (dx * dx + dy * dy) * fw;
-      if (dens) st += sqrt(ex * ex + ey * ey) * fw;
+      st += sqrt(ex * ex + ey * ey) * fw;
     }
   };
-  auto block4 = [&](const T (&raw)[4], int v) {
+  auto run = [&](const auto& raw, int v) {  // a run of ordinates from v
     double bp = 0, bt = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) term(raw[j], v + j, bp, bt);
+    for (int j = 0; j < (int)(sizeof(raw) / sizeof(T)); ++j) term(raw[j], v + j, bp, bt);
     if (kComp) {
       nsum<true>(sp, cp, bp);
-      if (dens) nsum<true>(st, ct, bt);
+      nsum<true>(st, ct, bt);
     }
   };
-  const int vper = ((V + S - 1) / S + 3) / 4 * 4;
+  constexpr int kB = 4;
+  const int vper = ((V + S - 1) / S + kB - 1) / kB * kB;
   const int vb = min(V, sub * vper), ve = min(V, vb + vper);
   int v = vb;
   if (live) {
-    // A ring of kMomRing register sets of four ordinates: while one set is
+    // A ring of kMomRing register sets of kB ordinates: while one set is
     // summed, the loads of the next sets are in flight.  Ring positions are
     // compile-time (unrolled), loads are clamped to the share's last
     // ordinate (none is conditional), and the sums run in ordinate order.
     constexpr int kR = kMomRing<T>;
-    if (ve - vb >= 4 * kR) {
-      T ring[kR][4];
+    if (ve - vb >= kB * kR) {
+      T ring[kR][kB];
 #pragma unroll
       for (int r = 0; r < kR; ++r)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) ring[r][j] = fload_nt(fp + (size_t)(vb + 4 * r + j) * a.ldf);
-      for (; v + 4 * kR <= ve; v += 4 * kR) {
+        for (int j = 0; j < kB; ++j) ring[r][j] = fload_nt(fp + (size_t)(vb + kB * r + j) * a.ldf);
+      for (; v + kB * kR <= ve; v += kB * kR) {
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-          T cur[4];
+          T cur[kB];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < kB; ++j) {
             cur[j] = ring[r][j];
-            ring[r][j] = fload_nt(fp + (size_t)min(v + 4 * (kR + r) + j, ve - 1) * a.ldf);
+            ring[r][j] = fload_nt(fp + (size_t)min(v + kB * (kR + r) + j, ve - 1) * a.ldf);
           }
-          block4(cur, v + 4 * r);
+          run(cur, v + kB * r);
         }
       }
-      // fewer than 4 kR ordinates remain; the ring holds them in order
+      // fewer than kB kR ordinates remain; the ring holds them in order
 #pragma unroll
       for (int r = 0; r < kR; ++r)
-        if (v + 4 <= ve) {
-          T cur[4];
+        if (v + kB <= ve) {
+          T cur[kB];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) cur[j] = ring[r][j];
-          block4(cur, v);
-          v += 4;
+          for (int j = 0; j < kB; ++j) cur[j] = ring[r][j];
+          run(cur, v);
+          v += kB;
         }
     }
-    for (; v + 4 <= ve; v += 4) {
-      T rc[4];
+    for (; v + kB <= ve; v += kB) {
+      T rc[kB];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) rc[j] = fp[(size_t)(v + j) * a.ldf];
-      block4(rc, v);
+      for (int j = 0; j < kB; ++j) rc[j] = fp[(size_t)(v + j) * a.ldf];
+      run(rc, v);
     }
     for (; v < ve; ++v) {
-      double bp = 0, bt = 0;
-      term(fp[(size_t)v * a.ldf], v, bp, bt);
-      if (kComp) {
-        nsum<true>(sp, cp, bp);
-        if (dens) nsum<true>(st, ct, bt);
-      }
+      const T rc[1] = {fp[(size_t)v * a.ldf]};
+      run(rc, v);
     }
   }
   double tp = sp, ep = cp, tt = st, et = ct;
@@ -1768,6 +1766,8 @@ int launch_moments(Ctx& c, bool sums, bool in_step) {
     hipLaunchKernelGGL((k_moments_once<T, 8>), g, dim3(512), 0, c.stream, m);
   else if (c.mom_once)
     hipLaunchKernelGGL((k_moments_once<T, 16>), g, dim3(1024), 0, c.stream, m);
+  else if (c.mom_split == 8)
+    hipLaunchKernelGGL((k_moments<T, 8>), g, dim3(512), 0, c.stream, m);
   else if (c.mom_split == 4)
     hipLaunchKernelGGL((k_moments<T, 4>), g, dim3(256), 0, c.stream, m);
   else if (c.mom_split == 2)
@@ -2461,18 +2461,25 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   const int wall_per = c.wall_ring ? 256 / p.T : 256;  // groups per block
   c.nblk_wall = nwe ? (nwe * c.ngroups + wall_per - 1) / wall_per : 0;
   // k_moments (k_moments_once keeps its own split): one wavefront per 64
-  // nodes leaves fewer than ~8 per SIMD
-  // below 512k nodes, and then up to four share each node's ordinates.  The
-  // choice depends on the node count only, so a mesh gives the same sums
-  // (and results) on any device.
+  // nodes leaves fewer than ~8 per SIMD below 512k nodes, and then up to
+  // eight share each node's ordinates.  Eight where four leave the chip's
+  // 8192 resident wavefronts unfilled and their shares stay longer than 64
+  // ordinates (us, four -> eight: 26,237 x 2048 FP32 185 -> 150, FP64 271 ->
+  // 265; 10,820 x 768 60 -> 40, 80 -> 59; 61,510 x 2048, 11536 wavefronts,
+  // 294 -> 306, 537 -> 555; 27,500 x 512 FP64 78 -> 83).  The choice depends
+  // on the node and ordinate counts only, so a mesh gives the same sums (and
+  // results) on any device.
   {
     const size_t n3 = 3 * (size_t)p.E;
-    if (!c.mom_once) c.mom_split = n3 < (size_t)1 << 19 ? 4 : (n3 < (size_t)1 << 20 ? 2 : 1);
+    if (!c.mom_once) {
+      c.mom_split = n3 < (size_t)1 << 19 ? 4 : (n3 < (size_t)1 << 20 ? 2 : 1);
+      if ((n3 + 63) / 64 * 4 < 8192 && p.V > 512) c.mom_split = 8;
+    }
     if (const char* ms = std::getenv("DGBGK_MOM_SPLIT")) {
       const int v = std::atoi(ms);
-      if (v == 1 || v == 2 || v == 4) c.mom_split = v;
+      if (v == 1 || v == 2 || v == 4 || v == 8) c.mom_split = v;
     }
-    const size_t per = c.mom_once ? 64 : 256 / c.mom_split;
+    const size_t per = c.mom_once ? 64 : std::max(64, 256 / c.mom_split);
     c.nblk_mom = (int)((n3 + per - 1) / per);
   }
   c.neta = (int)p.eta_side.size();

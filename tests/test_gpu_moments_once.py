@@ -1,7 +1,7 @@
 """The moments kernel that holds a node's ordinates in registers: shares of
 4, 8 and 16 wavefronts, full, ragged and shorter than a run of four, a
 wavefront without ordinates, the most it holds (512) and one more (513, the
-other kernel).  Against the FP64 CPU oracle: 1e-10 in FP64 (the same sums in
+other kernel's eight wavefronts per node).  Against the FP64 CPU oracle: 1e-10 in FP64 (the same sums in
 another order), 1e-5 in FP32."""
 import pytest
 
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("precision,tol", [(0, 1e-10), (1, 1e-5)])
 @pytest.mark.parametrize("rorder,torder,split", [
-    (6, 7, 4), (8, 16, 4), (3, 43, 8), (8, 32, 8), (3, 90, 16), (16, 32, 16), (27, 19, 4)])
+    (6, 7, 4), (8, 16, 4), (3, 43, 8), (8, 32, 8), (3, 90, 16), (16, 32, 16), (27, 19, 8)])
 def test_one_read_moments(rorder, torder, split, precision, tol):
     from dgbgk.solver import Solver
     from oracle_py import OracleRun
