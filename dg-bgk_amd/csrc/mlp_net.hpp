@@ -495,7 +495,9 @@ k_net(NetArgs a) {
 // wavefronts of W/2 x W/2 outputs.  The operands are stored as the MFMA
 // reads them (k_net), so they go from memory to registers; bound by reading
 // dZ and A once (67 MB a layer at 65,536 rows of width 256).  kPre pieces of
-// 16 rows are in flight per wavefront.
+// 16 rows are in flight per wavefront: 116 us for five such layers, 155 with
+// the loads left to the scheduler, which moves them to their use, and 147
+// with four blocks of a quarter of the outputs each, which read all twice.
 template <int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4)))
 k_wgrad(const uintx4* __restrict__ D, const uintx4* __restrict__ A, size_t act4, int rows_per,
@@ -517,26 +519,25 @@ k_wgrad(const uintx4* __restrict__ D, const uintx4* __restrict__ A, size_t act4,
 #pragma unroll
   for (int s = 0; s < kPre; ++s)
 #pragma unroll
-    for (int i = 0; i < M; ++i) {  // nb >= 2: rows_per is a multiple of 32
+    for (int i = 0; i < M; ++i) {  // nb is even: rows_per is a multiple of 32
       qd[s][i] = d[((size_t)s * NT + i) * 64];
       qa[s][i] = b[((size_t)s * NT + i) * 64];
     }
   for (int r = 0; r < nb; r += kPre) {
 #pragma unroll
     for (int s = 0; s < kPre; ++s) {
-      uintx4 cd[M], ca[M];
       const size_t rn = (size_t)min(r + s + kPre, nb - 1) * NT;
-#pragma unroll
-      for (int i = 0; i < M; ++i) {
-        cd[i] = qd[s][i];
-        ca[i] = qa[s][i];
-        qd[s][i] = d[(rn + i) * 64];
-        qa[s][i] = b[(rn + i) * 64];
-      }
 #pragma unroll
       for (int i = 0; i < M; ++i)
 #pragma unroll
-        for (int j = 0; j < M; ++j) acc[i][j] = mfma(cd[i], ca[j], acc[i][j]);
+        for (int j = 0; j < M; ++j) acc[i][j] = mfma(qd[s][i], qa[s][j], acc[i][j]);
+      // the set's registers are free again: its next piece, kPre on
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        qd[s][i] = d[(rn + i) * 64];
+        qa[s][i] = b[(rn + i) * 64];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay here, not at their use
     }
   }
   float* o = P + (l * gridDim.x + blockIdx.x) * (size_t)W * W;
@@ -551,7 +552,8 @@ k_wgrad(const uintx4* __restrict__ D, const uintx4* __restrict__ A, size_t act4,
 }
 
 // All partial sums of a step to the packed gradient: kRedCols outputs per
-// block, as k_reduce_splits.  Blocks: the hidden weights, the hidden
+// block, as k_reduce_splits, eight of a thread's partials in flight (46 -> 21
+// us for 84 MB; one after the other they were latency).  Blocks: the hidden weights, the hidden
 // biases, the input layer, the output layer.
 struct NetReduce {
   const float *pw, *pbias, *pin, *pout;
@@ -600,7 +602,16 @@ __global__ void __launch_bounds__(256) k_reduce_net(NetReduce a) {
   }
   float s = 0.0f;
   if (i < n)
-    for (int z = grp; z < splits; z += kRedGroups) s += P[(size_t)z * n + i];
+    for (int z = grp; z < splits; z += 8 * kRedGroups) {
+      float x[8];  // in flight together, added in order (past the end: 0)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int zj = z + j * kRedGroups;
+        x[j] = zj < splits ? P[(size_t)zj * n + i] : 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += x[j];
+    }
   s_sum[grp][c] = s;
   __syncthreads();
   if (grp != 0 || i >= n) return;
