@@ -26,6 +26,7 @@
 #include "../../include/dgbgk.h"
 #include "kernels.hpp"
 #include "prep.hpp"
+#include "staging.hpp"
 
 namespace dgbgk {
 
@@ -1598,29 +1599,32 @@ static __device__ __align__(256) double scratch[3 * kFstatsMaxBlocks + 4];
 // Layout conversions between the reference's DISNF(3,V,E) (double, input
 // element numbering) and the device's velocity-major T[V][ldf] (storage
 // order; eorder maps a storage position to its input element, or is null
-// when the two coincide).
+// when the two coincide), for input elements lo .. hi-1 (the array's first
+// element being lo).
 template <typename T>
 __global__ void k_to_device(const double* __restrict__ in, T* __restrict__ out,
-                            const int* __restrict__ eorder, int E, int V, long long ldf) {
+                            const int* __restrict__ eorder, int lo, int hi, int E, int V,
+                            long long ldf) {
   const size_t N3 = 3 * (size_t)E;
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int v = blockIdx.y;
   if (k >= N3) return;
-  const size_t e = k / 3, a = k % 3;
-  const size_t ei = eorder ? (size_t)eorder[e] : e;
-  out[(size_t)v * ldf + k] = (T)in[(ei * V + v) * 3 + a];
+  const int e = (int)(k / 3), a = (int)(k % 3), ei = eorder ? eorder[e] : e;
+  if (ei < lo || ei >= hi) return;
+  out[(size_t)v * ldf + k] = (T)in[((size_t)(ei - lo) * V + v) * 3 + a];
 }
 
 template <typename T>
 __global__ void k_to_host(const T* __restrict__ in, double* __restrict__ out,
-                          const int* __restrict__ eorder, int E, int V, long long ldf) {
+                          const int* __restrict__ eorder, int lo, int hi, int E, int V,
+                          long long ldf) {
   const size_t N3 = 3 * (size_t)E;
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int v = blockIdx.y;
   if (k >= N3) return;
-  const size_t e = k / 3, a = k % 3;
-  const size_t ei = eorder ? (size_t)eorder[e] : e;
-  out[(ei * V + v) * 3 + a] = (double)in[(size_t)v * ldf + k];
+  const int e = (int)(k / 3), a = (int)(k % 3), ei = eorder ? eorder[e] : e;
+  if (ei < lo || ei >= hi) return;
+  out[((size_t)(ei - lo) * V + v) * 3 + a] = (double)in[(size_t)v * ldf + k];
 }
 
 // ---------------------------------------------------------------------------
@@ -2183,8 +2187,8 @@ int upload_tables(Ctx& c) {
 
 template <typename T>
 int seed_points(Ctx& c, const std::vector<double>& ps4) {
-  HIPCK(hipMemcpyAsync(c.ps4, ps4.data(), ps4.size() * sizeof(double), hipMemcpyHostToDevice,
-                       c.stream));
+  HIPCK(stage_copy(c.ps4, const_cast<double*>(ps4.data()), ps4.size() * sizeof(double), true,
+                   c.stream, c.dev));
   const size_t N3 = 3 * (size_t)c.p.E;
   const dim3 g((unsigned)((N3 + 255) / 256), c.nvchunks);
   if (c.fuse_mom)
@@ -2207,6 +2211,36 @@ int refresh(Ctx& c, bool sums) {
   // DTE for the next step, no record
   HIPCK(hipMemsetAsync(c.res_part, 0, 2 * sizeof(double) * (c.nblk_upd + c.nblk_wall), c.stream));
   return launch_final(c, -1);
+}
+
+// f to or from the reference layout, through the f buffer that holds the
+// previous step (every element of it is rewritten by the next step before it
+// is read): as many input elements a pass as it holds as doubles.
+template <typename T>
+int transfer_f(Ctx& c, double* host, bool toDev) {
+  const int E = c.p.E, V = c.p.V;
+  const size_t N3 = 3 * (size_t)E;
+  const int per = (int)std::min<size_t>(E, c.ldf * sizeof(T) / (3 * sizeof(double)));
+  double* d = (double*)c.f[1 - c.cur];
+  T* f = (T*)c.f[c.cur];
+  const dim3 g((unsigned)((N3 + 255) / 256), V);
+  for (int lo = 0; lo < E; lo += per) {
+    const int hi = std::min(E, lo + per);
+    const size_t bytes = 3 * (size_t)(hi - lo) * V * sizeof(double);
+    double* part = host + 3 * (size_t)lo * V;
+    if (toDev) {
+      HIPCK(stage_copy(d, part, bytes, true, c.stream, c.dev));
+      hipLaunchKernelGGL(k_to_device<T>, g, dim3(256), 0, c.stream, d, f,
+                         (const int*)c.d_eorder, lo, hi, E, V, (long long)c.ldf);
+      HIPCK(hipGetLastError());
+    } else {
+      hipLaunchKernelGGL(k_to_host<T>, g, dim3(256), 0, c.stream, (const T*)f, d,
+                         (const int*)c.d_eorder, lo, hi, E, V, (long long)c.ldf);
+      HIPCK(hipGetLastError());
+      HIPCK(stage_copy(d, part, bytes, false, c.stream, c.dev));
+    }
+  }
+  return kOk;
 }
 
 int do_refresh(Ctx& c, bool sums) {
@@ -2518,6 +2552,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   if ((st = do_refresh(c, true))) return cleanup(st);
   if (hipStreamSynchronize(c.stream) != hipSuccess)
     return cleanup(fail(kErrHip, "initialisation failed on the device"));
+  StagePool::get().user(1);
   *out = h;
   return kOk;
 }
@@ -2535,6 +2570,7 @@ void dgbgk_destroy(dgbgk_ctx* h) {
     if (g) (void)hipGraphExecDestroy(g);
   for (void* q : c.owned) (void)hipFree(q);
   if (c.stream) (void)hipStreamDestroy(c.stream);
+  StagePool::get().user(-1);
   delete h;
 }
 
@@ -2549,14 +2585,20 @@ int dgbgk_step(dgbgk_ctx* h, int nsteps, dgbgk_step_info* info) {
     if (st) return st;
     c.itime += batch;
     if (info) {
+      static_assert(1024 * sizeof(StepRec) <= kStageBlock, "a batch's records fit a block");
+      StageBlock b;
+      char* to = b.p ? b.p : (char*)(info + done);
       const int n1 = std::min(batch, c.rec_cap - first);
-      HIPCK(hipMemcpyAsync(info + done, c.rec + first, n1 * sizeof(StepRec),
-                           hipMemcpyDeviceToHost, c.stream));
+      HIPCK(hipMemcpyAsync(to, c.rec + first, n1 * sizeof(StepRec), hipMemcpyDeviceToHost,
+                           c.stream));
       if (batch > n1)
-        HIPCK(hipMemcpyAsync(info + done + n1, c.rec, (batch - n1) * sizeof(StepRec),
+        HIPCK(hipMemcpyAsync(to + n1 * sizeof(StepRec), c.rec, (batch - n1) * sizeof(StepRec),
                              hipMemcpyDeviceToHost, c.stream));
+      HIPCK(hipStreamSynchronize(c.stream));
+      if (b.p) std::memcpy((void*)(info + done), b.p, batch * sizeof(StepRec));
+    } else {
+      HIPCK(hipStreamSynchronize(c.stream));
     }
-    HIPCK(hipStreamSynchronize(c.stream));
     tharvest(c);
     done += batch;
   }
@@ -2565,47 +2607,16 @@ int dgbgk_step(dgbgk_ctx* h, int nsteps, dgbgk_step_info* info) {
 
 int dgbgk_get_f(dgbgk_ctx* h, double* f) {
   if (!h || !f) return fail(kErrArg, "null argument");
-  Ctx& c = h->c;
-  const size_t n = 3 * (size_t)c.p.E * c.p.V;
-  double* d = nullptr;
-  HIPCK(hipMalloc((void**)&d, n * sizeof(double)));
-  const size_t N3 = 3 * (size_t)c.p.E;
-  dim3 g((unsigned)((N3 + 255) / 256), c.p.V);
-  if (c.prec)
-    hipLaunchKernelGGL(k_to_host<float>, g, dim3(256), 0, c.stream, (const float*)c.f[c.cur], d,
-                       (const int*)c.d_eorder, c.p.E, c.p.V, (long long)c.ldf);
-  else
-    hipLaunchKernelGGL(k_to_host<double>, g, dim3(256), 0, c.stream,
-                       (const double*)c.f[c.cur], d, (const int*)c.d_eorder, c.p.E, c.p.V,
-                       (long long)c.ldf);
-  hipError_t e1 = hipMemcpyAsync(f, d, n * sizeof(double), hipMemcpyDeviceToHost, c.stream);
-  hipError_t e2 = hipStreamSynchronize(c.stream);
-  const hipError_t e3 = hipFree(d);
-  if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) return fail(kErrHip, "get_f failed");
-  return kOk;
+  return h->c.prec ? transfer_f<float>(h->c, f, false) : transfer_f<double>(h->c, f, false);
 }
 
 int dgbgk_set_f(dgbgk_ctx* h, const double* f) {
   if (!h || !f) return fail(kErrArg, "null argument");
   Ctx& c = h->c;
-  const size_t n = 3 * (size_t)c.p.E * c.p.V;
-  double* d = nullptr;
-  HIPCK(hipMalloc((void**)&d, n * sizeof(double)));
-  hipError_t e1 = hipMemcpyAsync(d, f, n * sizeof(double), hipMemcpyHostToDevice, c.stream);
-  const size_t N3 = 3 * (size_t)c.p.E;
-  dim3 g((unsigned)((N3 + 255) / 256), c.p.V);
-  if (c.prec)
-    hipLaunchKernelGGL(k_to_device<float>, g, dim3(256), 0, c.stream, d, (float*)c.f[c.cur],
-                       (const int*)c.d_eorder, c.p.E, c.p.V, (long long)c.ldf);
-  else
-    hipLaunchKernelGGL(k_to_device<double>, g, dim3(256), 0, c.stream, d,
-                       (double*)c.f[c.cur], (const int*)c.d_eorder, c.p.E, c.p.V,
-                       (long long)c.ldf);
-  int st = do_refresh(c, false);
-  hipError_t e2 = hipStreamSynchronize(c.stream);
-  const hipError_t e3 = hipFree(d);
-  if (st) return st;
-  if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) return fail(kErrHip, "set_f failed");
+  double* src = const_cast<double*>(f);  // read only
+  int st = c.prec ? transfer_f<float>(c, src, true) : transfer_f<double>(c, src, true);
+  if (st || (st = do_refresh(c, false))) return st;
+  HIPCK(hipStreamSynchronize(c.stream));
   return kOk;
 }
 
@@ -2659,11 +2670,22 @@ int dgbgk_point_fields(dgbgk_ctx* h, double* nd, double* rho, double* uvel, doub
   if (st) return st;
   const size_t P = c.p.P;
   double* dst[6] = {nd, rho, uvel, vvel, ps, temp};
-  for (int i = 0; i < 6; ++i)
-    if (dst[i])
-      HIPCK(hipMemcpyAsync(dst[i], c.pts + i * P, P * sizeof(double), hipMemcpyDeviceToHost,
-                           c.stream));
-  HIPCK(hipStreamSynchronize(c.stream));
+  int i0 = 0, i1 = 6;  // the rows asked for
+  while (i0 < 6 && !dst[i0]) ++i0;
+  while (i1 > i0 && !dst[i1 - 1]) --i1;
+  const size_t row = P * sizeof(double);
+  if ((i1 - i0) * row <= kStageBlock) {  // all in one copy
+    StageBlock b;
+    if (b.p) {
+      HIPCK(hipMemcpyAsync(b.p, c.pts + i0 * P, (i1 - i0) * row, hipMemcpyDeviceToHost, c.stream));
+      HIPCK(hipStreamSynchronize(c.stream));
+      for (int i = i0; i < i1; ++i)
+        if (dst[i]) std::memcpy(dst[i], b.p + (i - i0) * row, row);
+      return kOk;
+    }
+  }
+  for (int i = i0; i < i1; ++i)
+    if (dst[i]) HIPCK(stage_copy(c.pts + i * P, dst[i], row, false, c.stream, c.dev));
   return kOk;
 }
 
