@@ -11,7 +11,8 @@
 //   k_moments_once  compensated in FP32
 //   k_points   point averages (GETMAC) when the reference gathers them
 //   k_final    residual max, mass, forces, next DTE (ALOTIM2); with
-//              k_moments_once by that launch's last block
+//              k_moments_once only after a batch's last step: the others'
+//              epilogues are a block of the next step's k_update
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -183,6 +184,27 @@ __device__ __forceinline__ double block_max(double x, double* sh) {
     for (int i = 1; i < nw; ++i) x = fmax(x, sh[i]);
   }
   return x;  // valid in thread 0
+}
+
+// Both maxima in one round; sh: two doubles per wavefront.
+__device__ __forceinline__ double2 block_max2(double x, double y, double* sh) {
+  for (int o = 32; o > 0; o >>= 1) {
+    x = fmax(x, __shfl_down(x, o, 64));
+    y = fmax(y, __shfl_down(y, o, 64));
+  }
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, nw = (blockDim.x + 63) >> 6;
+  __syncthreads();
+  if (l == 0) {
+    sh[w] = x;
+    sh[nw + w] = y;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int i = 1; i < nw; ++i) {
+      x = fmax(x, sh[i]);
+      y = fmax(y, sh[nw + i]);
+    }
+  return make_double2(x, y);  // valid in thread 0
 }
 
 __device__ __forceinline__ double block_sum(double x, double* sh) {
@@ -462,6 +484,177 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
   }
 }
 
+// GETMAC runs on every 1000th step (src/advnce.f90:403-406).
+__device__ __forceinline__ bool gather_step(double steps_done) {
+  return ((long long)steps_done + 1) % 1000 == 0;
+}
+
+// MACROS point averages (src/macros.f90:156-188) of point q over the point
+// CSR; gather: also GETMAC's copy of the pressure for GETFOR.
+__device__ __forceinline__ void point_average(int q, const double* __restrict__ mom,
+                                              const double* __restrict__ rj,
+                                              const int* __restrict__ ptr,
+                                              const int* __restrict__ node,
+                                              double* __restrict__ pts,
+                                              double* __restrict__ ps_glob, int E, int P,
+                                              double mm, double rgas, int gather) {
+  const size_t N3 = 3 * (size_t)E;
+  double flag = 0, nd = 0, u = 0, vv = 0, ps = 0;
+  for (int i = ptr[q]; i < ptr[q + 1]; ++i) {
+    const int k = node[i];
+    const double ae = rj[k / 3];
+    const double n = mom[k];
+    if (n >= 1e-20) {
+      u += ae * mom[N3 + k];
+      vv += ae * mom[2 * N3 + k];
+    }
+    flag += ae;
+    nd += n * ae;
+    ps += mom[3 * N3 + k] * ae;
+  }
+  double rho = 0, t = 0;
+  if (nd < 1e-20) {
+    u = vv = ps = 0.0;
+  } else {
+    nd = nd / flag;
+    rho = nd * mm;
+    u = u / flag;
+    vv = vv / flag;
+    ps = ps / flag;
+    t = ps / (rgas * rho);
+  }
+  pts[q] = nd;
+  pts[P + q] = rho;
+  pts[2 * P + q] = u;
+  pts[3 * P + q] = vv;
+  pts[4 * P + q] = ps;
+  pts[5 * P + q] = t;
+  if (gather) ps_glob[q] = ps;
+}
+
+// ALOTIM2 (src/alotim2.f90): the next step's DTE from the largest MU
+__device__ __forceinline__ double next_dte(double m, double cap) {
+  const double dteb = (m > 0.0) ? 0.9 * (1 / m) : 1000000.0;
+  return dteb < cap ? dteb : cap;
+}
+
+// Step epilogue: GETRES max, mass, GETFOR (src/getfor.f90:29-49) on the
+// gathered point pressure, the residual record, and ALOTIM2's next DTE, by
+// one block of at most 1024 threads.
+__device__ __forceinline__ void final_body(const FinalArgs& a, double (&s_red)[6][16]) {
+  double* const scal = a.scal;
+  const double steps_done = scal[6] + a.ahead;  // in flight with the partials below
+  double r = 0.0, rc = 0.0, m = 0.0, ms = 0.0, lift = 0.0, drag = 0.0;
+  // each thread's partials, up to kLd per array loaded before any is
+  // combined (one memory latency instead of one per partial); combined in
+  // index order, so the mass sum keeps its order (out-of-range slots add
+  // 0 and all partials are >= 0)
+  constexpr int kLd = 8;
+  const int nt = blockDim.x, nres = a.nres, nmom = a.nmom;
+  for (int b = threadIdx.x; b < nres; b += kLd * nt) {
+    double x[kLd], y[kLd];
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      const int i = b + j * nt;
+      x[j] = i < nres ? a.res_part[i] : 0.0;
+      y[j] = i < nres ? a.res_part[nres + i] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      r = fmax(r, x[j]);
+      rc = fmax(rc, y[j]);
+    }
+  }
+  for (int b = threadIdx.x; b < nmom; b += kLd * nt) {
+    double x[kLd], y[kLd];
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      const int i = b + j * nt;
+      x[j] = i < nmom ? a.mu_part[i] : 0.0;
+      y[j] = i < nmom ? a.mass_part[i] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < kLd; ++j) {
+      m = fmax(m, x[j]);
+      ms += y[j];
+    }
+  }
+  // In a step, GETMAC on every 1000th step (src/advnce.f90:403-406): the
+  // point averages and the gathered pressure that GETFOR below uses.  Rare,
+  // so this block does it rather than a launch every step.
+  if (a.record >= 0 && gather_step(steps_done)) {
+    for (int q = threadIdx.x; q < a.P; q += blockDim.x)
+      point_average(q, a.mom, a.rj, a.ptr, a.node, a.pts, a.ps_glob, a.E, a.P, a.mm, a.rgas, 1);
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < a.nf; i += blockDim.x) {
+    const int p1 = a.fside[2 * i], p2 = a.fside[2 * i + 1];
+    const double x1 = a.coord[2 * p1], y1 = a.coord[2 * p1 + 1];
+    const double x2 = a.coord[2 * p2], y2 = a.coord[2 * p2 + 1];
+    const double len = sqrt((x2 - x1) * (x2 - x1) + (y2 - y1) * (y2 - y1));
+    const double px = -(y2 - y1), py = x2 - x1;
+    const double mag = sqrt(px * px + py * py);
+    const double psav = 0.5 * (a.ps_glob[p1] + a.ps_glob[p2]);
+    lift -= psav * len * (py / mag);
+    drag -= psav * len * (px / mag);
+  }
+  // the three maxima and three sums in one LDS round: each wavefront
+  // reduces its six values, then thread j combines value j over the
+  // wavefronts in wavefront order (the order of block_max / block_sum)
+  for (int o = 32; o > 0; o >>= 1) {
+    r = fmax(r, __shfl_down(r, o, 64));
+    rc = fmax(rc, __shfl_down(rc, o, 64));
+    m = fmax(m, __shfl_down(m, o, 64));
+    ms += __shfl_down(ms, o, 64);
+    lift += __shfl_down(lift, o, 64);
+    drag += __shfl_down(drag, o, 64);
+  }
+  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    s_red[0][w] = r;
+    s_red[1][w] = rc;
+    s_red[2][w] = m;
+    s_red[3][w] = ms;
+    s_red[4][w] = lift;
+    s_red[5][w] = drag;
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int j = threadIdx.x;
+    double x = s_red[j][0];
+    for (int i = 1; i < nw; ++i) x = j < 3 ? fmax(x, s_red[j][i]) : x + s_red[j][i];
+    s_red[j][0] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    r = s_red[0][0];
+    rc = s_red[1][0];
+    m = s_red[2][0];
+    ms = s_red[3][0];
+    lift = s_red[4][0];
+    drag = s_red[5][0];
+    if (a.record >= 0) {
+      // scal[6] counts the steps completed when the batch began (ITIME of
+      // src/advnce.f90:220 between batches)
+      const long long itime = (long long)steps_done + 1;
+      if (a.end) scal[6] = (double)itime;
+      const int slot = (int)((itime - 1) % a.rec_cap);
+      if (itime == 1) scal[1] = r;
+      a.rec[slot].sumres = r;
+      a.rec[slot].logres = log(r / scal[1]);
+      a.rec[slot].dte = scal[0];
+      a.rec[slot].mass = ms;
+      a.rec[slot].lift = lift;
+      a.rec[slot].drag = drag;
+      a.rec[slot].change = rc;
+    }
+    scal[2] = lift;
+    scal[3] = drag;
+    scal[5] = ms;
+    scal[0] = next_dte(m, scal[4]);
+  }
+}
+
 // FLUCON2 (src/flucon2.f90:133-233) of type-4 wall side j by the first 256
 // threads of one of the update launch's leading blocks: the wall pass that
 // follows needs it, the update does not, and a launch of its own took 5 us
@@ -515,12 +708,21 @@ k_update(UpdArgs<T> a) {
   __shared__ __align__(16) T s_f[kQ][kRow];
   if (sizeof(T) == 4 && threadIdx.x < 4 * kQ)  // read after the first barrier
     s_f[threadIdx.x / 4][kS * 4 + threadIdx.x % 4] = T(0);
-  __shared__ double s_red[8];
+  __shared__ double s_red[6][16];
   if ((int)blockIdx.x < a.neta) {
-    wall_eta(a, blockIdx.x, s_red);
+    wall_eta(a, blockIdx.x, s_red[0]);
     return;
   }
-  const int logical = xcd_logical(blockIdx.x - a.neta, gridDim.x - a.neta);
+  // A step whose predecessor left its epilogue to this launch: one block does
+  // it, and every other forms DTE itself, from the moments' partial maxima
+  // (1 us with the tables' loads under way).  On its own between two steps the
+  // epilogue takes 6 us.
+  const int lead = a.neta + (kMom ? 0 : a.pending);
+  if (!kMom && (int)blockIdx.x < lead) {
+    final_body(a.fin, s_red);
+    return;
+  }
+  const int logical = xcd_logical(blockIdx.x - lead, gridDim.x - lead);
   const int tile = logical % a.ntiles;
   const int v0 = (logical / a.ntiles) * a.vchunk;
   const int v1 = min(a.V, v0 + a.vchunk);
@@ -535,7 +737,30 @@ k_update(UpdArgs<T> a) {
   s.active = slot < nown + nh;
   s.e = s.owned ? e0 + slot : (s.active ? a.halo[hoff + slot - nown] : 0);
   const int e = s.e;
-  const T dte = (T)a.scal[0];
+  double dt;
+  if (!kMom && a.pending) {
+    constexpr int kLd = 8;
+    double m = 0.0;
+    for (int b = slot; b < a.fin.nmom; b += kLd * kS) {
+      double x[kLd];
+#pragma unroll
+      for (int j = 0; j < kLd; ++j) {
+        const int i = b + j * kS;
+        x[j] = i < a.fin.nmom ? a.fin.mu_part[i] : 0.0;
+      }
+#pragma unroll
+      for (int j = 0; j < kLd; ++j) m = fmax(m, x[j]);
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if ((slot & 63) == 0) s_red[0][slot >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kS / 64; ++w) m = fmax(m, s_red[0][w]);
+    dt = next_dte(m, a.scal[4]);
+  } else {
+    dt = a.scal[0];
+  }
+  const T dte = (T)dt;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     s.gx[k] = s.gy[k] = s.pA[k] = s.pB[k] = s.pU[k] = s.pV[k] = s.pMd[k] = T(0);
@@ -587,7 +812,7 @@ k_update(UpdArgs<T> a) {
   }
   T res = 0, chg = 0;
 
-  const double stw = a.scal[6] * 0.6180339887498949;  // Weyl step phase
+  const double stw = (a.scal[6] + a.ahead) * 0.6180339887498949;  // Weyl step phase
   const float sph = (float)(stw - floor(stw));
   const float dsc0 = a.dither ? 0x1p-23f : 0.f, dsc1 = a.dither ? -0x1p-24f : 0.f;
   const bool anyin = __ballot(s.mask != 0) != 0;
@@ -637,10 +862,11 @@ k_update(UpdArgs<T> a) {
       ms[2 * N3 + k] = m2[k];
     }
   }
-  const double r = block_max((double)res, s_red);
-  if (threadIdx.x == 0) a.res_part[logical] = r;
-  const double rc = block_max((double)chg, s_red);
-  if (threadIdx.x == 0) a.res_part[a.res_stride + logical] = rc;
+  const double2 r = block_max2((double)res, (double)chg, s_red[0]);
+  if (threadIdx.x == 0) {
+    a.res_part[logical] = r.x;
+    a.res_part[a.res_stride + logical] = r.y;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -676,7 +902,7 @@ struct WallElem {
     mask = a.emask[e];
     // FP32 store dither (as in k_update): element, ordinate and step phases
     wph = a.ephase[e];
-    const double stw = a.scal[6] * 0.6180339887498949;
+    const double stw = (a.scal[6] + a.ahead) * 0.6180339887498949;
     sph = (float)(stw - floor(stw));
   }
 };
@@ -904,182 +1130,6 @@ __global__ void __launch_bounds__(256) k_wall_ring(WallArgs<T> a) {
   if (threadIdx.x == 0) a.res_part[blockIdx.x] = r;
   const double rc = block_max(chg, s_red);
   if (threadIdx.x == 0) a.res_part[a.res_stride + blockIdx.x] = rc;
-}
-
-// Loads and stores past this XCD's caches, for values that blocks of one
-// launch on different XCDs exchange.
-__device__ __forceinline__ double agent_load(const double* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void agent_store(double* p, double x) {
-  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// GETMAC runs on every 1000th step (src/advnce.f90:403-406).
-__device__ __forceinline__ bool gather_step(double steps_done) {
-  return ((long long)steps_done + 1) % 1000 == 0;
-}
-
-// MACROS point averages (src/macros.f90:156-188) of point q over the point
-// CSR; gather: also GETMAC's copy of the pressure for GETFOR.
-__device__ __forceinline__ void point_average(int q, const double* __restrict__ mom,
-                                              const double* __restrict__ rj,
-                                              const int* __restrict__ ptr,
-                                              const int* __restrict__ node,
-                                              double* __restrict__ pts,
-                                              double* __restrict__ ps_glob, int E, int P,
-                                              double mm, double rgas, int gather) {
-  const size_t N3 = 3 * (size_t)E;
-  double flag = 0, nd = 0, u = 0, vv = 0, ps = 0;
-  for (int i = ptr[q]; i < ptr[q + 1]; ++i) {
-    const int k = node[i];
-    const double ae = rj[k / 3];
-    const double n = mom[k];
-    if (n >= 1e-20) {
-      u += ae * mom[N3 + k];
-      vv += ae * mom[2 * N3 + k];
-    }
-    flag += ae;
-    nd += n * ae;
-    ps += mom[3 * N3 + k] * ae;
-  }
-  double rho = 0, t = 0;
-  if (nd < 1e-20) {
-    u = vv = ps = 0.0;
-  } else {
-    nd = nd / flag;
-    rho = nd * mm;
-    u = u / flag;
-    vv = vv / flag;
-    ps = ps / flag;
-    t = ps / (rgas * rho);
-  }
-  pts[q] = nd;
-  pts[P + q] = rho;
-  pts[2 * P + q] = u;
-  pts[3 * P + q] = vv;
-  pts[4 * P + q] = ps;
-  pts[5 * P + q] = t;
-  if (gather) ps_glob[q] = ps;
-}
-
-// Step epilogue: GETRES max, mass, GETFOR (src/getfor.f90:29-49) on the
-// gathered point pressure, the residual record, and ALOTIM2's next DTE, by
-// one block of at most 1024 threads.
-__device__ __forceinline__ void final_body(const FinalArgs& a, double (&s_red)[6][16]) {
-  double* const scal = a.scal;
-  const double steps_done = scal[6];  // in flight with the partials below
-  double r = 0.0, rc = 0.0, m = 0.0, ms = 0.0, lift = 0.0, drag = 0.0;
-  // each thread's partials, up to kLd per array loaded before any is
-  // combined (one memory latency instead of one per partial); combined in
-  // index order, so the mass sum keeps its order (out-of-range slots add
-  // 0 and all partials are >= 0)
-  constexpr int kLd = 8;
-  const int nt = blockDim.x, nres = a.nres, nmom = a.nmom;
-  for (int b = threadIdx.x; b < nres; b += kLd * nt) {
-    double x[kLd], y[kLd];
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      const int i = b + j * nt;
-      x[j] = i < nres ? a.res_part[i] : 0.0;
-      y[j] = i < nres ? a.res_part[nres + i] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      r = fmax(r, x[j]);
-      rc = fmax(rc, y[j]);
-    }
-  }
-  // (agent scope: the moments launch that ends with this may have written
-  // them from other XCDs)
-  for (int b = threadIdx.x; b < nmom; b += kLd * nt) {
-    double x[kLd], y[kLd];
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      const int i = b + j * nt;
-      x[j] = i < nmom ? agent_load(a.mu_part + i) : 0.0;
-      y[j] = i < nmom ? agent_load(a.mass_part + i) : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kLd; ++j) {
-      m = fmax(m, x[j]);
-      ms += y[j];
-    }
-  }
-  // In a step, GETMAC on every 1000th step (src/advnce.f90:403-406): the
-  // point averages and the gathered pressure that GETFOR below uses.  Rare,
-  // so this block does it rather than a launch every step.
-  if (a.record >= 0 && gather_step(steps_done)) {
-    for (int q = threadIdx.x; q < a.P; q += blockDim.x)
-      point_average(q, a.mom, a.rj, a.ptr, a.node, a.pts, a.ps_glob, a.E, a.P, a.mm, a.rgas, 1);
-    __syncthreads();
-  }
-  for (int i = threadIdx.x; i < a.nf; i += blockDim.x) {
-    const int p1 = a.fside[2 * i], p2 = a.fside[2 * i + 1];
-    const double x1 = a.coord[2 * p1], y1 = a.coord[2 * p1 + 1];
-    const double x2 = a.coord[2 * p2], y2 = a.coord[2 * p2 + 1];
-    const double len = sqrt((x2 - x1) * (x2 - x1) + (y2 - y1) * (y2 - y1));
-    const double px = -(y2 - y1), py = x2 - x1;
-    const double mag = sqrt(px * px + py * py);
-    const double psav = 0.5 * (a.ps_glob[p1] + a.ps_glob[p2]);
-    lift -= psav * len * (py / mag);
-    drag -= psav * len * (px / mag);
-  }
-  // the three maxima and three sums in one LDS round: each wavefront
-  // reduces its six values, then thread j combines value j over the
-  // wavefronts in wavefront order (the order of block_max / block_sum)
-  for (int o = 32; o > 0; o >>= 1) {
-    r = fmax(r, __shfl_down(r, o, 64));
-    rc = fmax(rc, __shfl_down(rc, o, 64));
-    m = fmax(m, __shfl_down(m, o, 64));
-    ms += __shfl_down(ms, o, 64);
-    lift += __shfl_down(lift, o, 64);
-    drag += __shfl_down(drag, o, 64);
-  }
-  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    s_red[0][w] = r;
-    s_red[1][w] = rc;
-    s_red[2][w] = m;
-    s_red[3][w] = ms;
-    s_red[4][w] = lift;
-    s_red[5][w] = drag;
-  }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int j = threadIdx.x;
-    double x = s_red[j][0];
-    for (int i = 1; i < nw; ++i) x = j < 3 ? fmax(x, s_red[j][i]) : x + s_red[j][i];
-    s_red[j][0] = x;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    r = s_red[0][0];
-    rc = s_red[1][0];
-    m = s_red[2][0];
-    ms = s_red[3][0];
-    lift = s_red[4][0];
-    drag = s_red[5][0];
-    if (a.record >= 0) {
-      // scal[6] counts completed steps (ITIME of src/advnce.f90:220)
-      const long long itime = (long long)scal[6] + 1;
-      scal[6] = (double)itime;
-      const int slot = (int)((itime - 1) % a.rec_cap);
-      if (itime == 1) scal[1] = r;
-      a.rec[slot].sumres = r;
-      a.rec[slot].logres = log(r / scal[1]);
-      a.rec[slot].dte = scal[0];
-      a.rec[slot].mass = ms;
-      a.rec[slot].lift = lift;
-      a.rec[slot].drag = drag;
-      a.rec[slot].change = rc;
-    }
-    scal[2] = lift;
-    scal[3] = drag;
-    scal[5] = ms;
-    const double dteb = (m > 0.0) ? 0.9 * (1 / m) : 1000000.0;
-    scal[0] = dteb < scal[4] ? dteb : scal[4];
-  }
 }
 
 __global__ void __launch_bounds__(1024) k_final(FinalArgs a) {
@@ -1345,76 +1395,108 @@ __global__ void __launch_bounds__(S > 4 ? 64 * S : 256) k_moments(MomArgs<T> a) 
   if (threadIdx.x == 0) a.mass_part[blockIdx.x] = m2;
 }
 
-// k_moments_once: the same sums where a block's wavefronts hold all V
-// ordinates of 64 nodes in registers (at most kMomHold each), so f is read
-// once, the update leaves no partial sums, and every load of the kernel is
-// in flight at the start.  For meshes whose step is bound by latency:
-// k_moments' rounds of loads (the update's sums, then f) take 26 us at 1,679
-// triangles x 128 in FP64 and 21 us at 5,763 x 128, this 10 and 14, and the
-// update 11 and 18 us against 15 and 21 with its sums.
+// k_moments_once: the same sums where a block's S wavefronts hold all V
+// ordinates of its nodes in registers, so f is read once, the update leaves no
+// partial sums, and every load of the kernel is in flight at the start.  For
+// meshes whose step is bound by latency: k_moments' rounds of loads (the
+// update's sums, then f) take 26 us at 1,679 triangles x 128 in FP64 and 21 us
+// at 5,763 x 128, this 10 and 14, and the update 11 and 18 us against 15 and
+// 21 with its sums.
+// L = 1: a lane per node and scalar loads of the velocity tables.  L = 4: four
+// lanes share a node's ordinates, so a block has 16 nodes (a row of 128 bytes)
+// and a quarter of the serial work, and the tables, whose rows then differ
+// between lanes, come from LDS.  A block's second pass alone took 4 of the 17
+// us at 5,763 x 128 with one wavefront per SIMD.
+// Nothing follows the blocks' partial results: that its last block ran the
+// step's epilogue cost 10 ns a block in counting them and 4 us of loads and
+// reductions behind them (5,763 x 128, a step: 38.6 us, 35.3 without).
 constexpr int kMomHold = 32;
 
-template <typename T, int S>
-__global__ void __launch_bounds__(64 * S) k_moments_once(MomArgs<T> a) {
+template <typename T, int S, int L>
+__global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(L > 1 ? 8 : 1, 8)))
+k_moments_once(MomArgs<T> a) {
   constexpr bool kComp = sizeof(T) < sizeof(double);
-  __shared__ double s_part[S][3][64];
-  __shared__ double s_red[6][16];
-  __shared__ int s_last;
-  const int lane = threadIdx.x & 63;
-  const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const size_t N3 = 3 * (size_t)a.E, k = (size_t)blockIdx.x * 64 + lane;
+  constexpr int N = 64 / L, H = kMomHold / L;
+  static_assert(L == 1 || !kComp, "FP32 takes the scalar tables");
+  __shared__ double s_tab[L > 1 ? 7 : 1][L > 1 ? kMomHold * S : 1];
+  __shared__ double s_part[S][3][N];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, node = lane % N, sub = wave * L + lane / N;
+  const size_t N3 = 3 * (size_t)a.E, k = (size_t)blockIdx.x * N + node;
   const bool live = k < N3;
-  const int V = a.V, vper = (V + S - 1) / S;
-  const int vb = min(V, sub * vper), cnt = min(V, vb + vper) - vb;
-  const T* fp = a.f + (live ? k : 0);
-  T f[kMomHold];
+  const int V = a.V, vper = (V + S * L - 1) / (S * L), vb = sub * vper;
+  const T* fp = a.f + (live ? k : 0) + (size_t)min(vb, V - 1) * a.ldf;
+  T f[H];
 #pragma unroll
-  for (int j = 0; j < kMomHold; j += 4)  // past the share: its last ordinate, unused
-    if (j < cnt) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        f[j + i] = fload_nt(fp + (size_t)(vb + min(j + i, cnt - 1)) * a.ldf);
+  for (int j = 0; j < H; ++j)
+    if (j < vper) {
+      f[j] = fload_nt(fp);
+      fp += vb + j + 1 < V ? a.ldf : 0;
     }
-  const double* cxa = a.vtd + vb;
-  const double* cya = a.vtd + V + vb;
-  const double* cxb = a.vtd + 2 * V + vb;
-  const double* cyb = a.vtd + 3 * V + vb;
-  const double* wv = a.vtd + 4 * V + vb;
-  const double* wcx = a.vtd + 5 * V + vb;
-  const double* wcy = a.vtd + 6 * V + vb;
-  const double* hv = a.vtd + 7 * V + vb;
-  const T* vt = a.vtab + vb;
-  // in runs of four ordinates (one set of scalar loads), then one by one
+  // Rows of the velocity tables: w, w c, c, and h (FP32, c as floats) or the
+  // adjacent c.
+  const int cnt = min(V, vb + vper) - vb;
+  if constexpr (L > 1) {
+    // zeros past V, where the last shares end (at most at kMomHold S)
+    for (int v = threadIdx.x; v < S * L * vper; v += 64 * S)
+#pragma unroll
+      for (int i = 0; i < 7; ++i) s_tab[i][v] = v < V ? a.vtd[(i < 3 ? 4 + i : i - 3) * V + v] : 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < H; ++j)
+      if (j >= cnt) f[j] = T(0);
+  }
+  auto tab = [&](int i, int j) -> double {
+    if constexpr (L > 1) return s_tab[i][vb + j];
+    if constexpr (kComp)
+      if (i == 3 || i == 4) return (double)ldc(a.vtab + (i - 3) * V + vb, j);
+    return ldc(a.vtd + (i < 3 ? 4 + i : (kComp ? 7 : i - 3)) * V + vb, j);
+  };
+  // the share's ordinates; scalar loads in runs of four, then one by one
   auto each = [&](auto&& body) {
+    if constexpr (L > 1) {
 #pragma unroll
-    for (int j = 0; j < kMomHold; j += 4) {
-      if (j + 4 <= cnt) {
+      for (int j = 0; j < H; ++j)
+        if (j < vper) body(j);
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) body(j + i);
-      } else {
+      for (int j = 0; j < H; j += 4) {
+        if (j + 4 <= cnt) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-          if (j + i < cnt) body(j + i);
+          for (int i = 0; i < 4; ++i) body(j + i);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            if (j + i < cnt) body(j + i);
+        }
       }
     }
   };
   double b0 = 0, b1 = 0, b2 = 0;
   each([&](int j) {
     const double fd = (double)f[j];
-    b0 = fma(ldc(wv, j), fd, b0);
-    b1 = fma(ldc(wcx, j), fd, b1);
-    b2 = fma(ldc(wcy, j), fd, b2);
+    b0 = fma(tab(0, j), fd, b0);
+    b1 = fma(tab(1, j), fd, b1);
+    b2 = fma(tab(2, j), fd, b2);
   });
-  s_part[sub][0][lane] = b0;
-  s_part[sub][1][lane] = b1;
-  s_part[sub][2][lane] = b2;
+#pragma unroll
+  for (int o = N; o < 64; o *= 2) {
+    b0 += __shfl_xor(b0, o, 64);
+    b1 += __shfl_xor(b1, o, 64);
+    b2 += __shfl_xor(b2, o, 64);
+  }
+  if (lane < N) {
+    s_part[wave][0][node] = b0;
+    s_part[wave][1][node] = b1;
+    s_part[wave][2][node] = b2;
+  }
   __syncthreads();
   double t0 = 0, e0 = 0, t1 = 0, e1 = 0, t2 = 0, e2 = 0;
 #pragma unroll
   for (int i = 0; i < S; ++i) {
-    nsum<kComp>(t0, e0, s_part[i][0][lane]);
-    nsum<kComp>(t1, e1, s_part[i][1][lane]);
-    nsum<kComp>(t2, e2, s_part[i][2][lane]);
+    nsum<kComp>(t0, e0, s_part[i][0][node]);
+    nsum<kComp>(t1, e1, s_part[i][1][node]);
+    nsum<kComp>(t2, e2, s_part[i][2][node]);
   }
   const double n = t0 - e0;
   const bool dens = n >= 1e-20;
@@ -1423,62 +1505,50 @@ __global__ void __launch_bounds__(64 * S) k_moments_once(MomArgs<T> a) {
   double bp = 0, bt = 0;  // the terms of k_moments' second pass
   each([&](int j) {
     if constexpr (kComp) {
-      const float ex = uxf - (float)ldc(vt, j), ey = uyf - (float)ldc(vt + V, j);
+      const float ex = uxf - (float)tab(3, j), ey = uyf - (float)tab(4, j);
       const float rel = __builtin_amdgcn_sqrtf(fmaf(ex, ex, ey * ey));
-      bp = fma((double)f[j], ldc(hv, j), bp);
-      bt = fma((double)(rel * (float)f[j]), ldc(wv, j), bt);
+      bp = fma((double)f[j], tab(5, j), bp);
+      bt = fma((double)(rel * (float)f[j]), tab(0, j), bt);
     } else {
-      const double fw = (double)f[j] * ldc(wv, j);
-      const double dx = ldc(cxb, j) - ux, dy = ldc(cyb, j) - uy;
-      const double ex = ux - ldc(cxa, j), ey = uy - ldc(cya, j);
+      const double fw = (double)f[j] * tab(0, j);
+      const double dx = tab(5, j) - ux, dy = tab(6, j) - uy;
+      const double ex = ux - tab(3, j), ey = uy - tab(4, j);
       bp += 0.5 * (dx * dx + dy * dy) * fw;
       bt += sqrt(ex * ex + ey * ey) * fw;
     }
   });
-  __syncthreads();  // every wavefront has read the first sums
-  s_part[sub][0][lane] = bp;
-  s_part[sub][1][lane] = bt;
-  __syncthreads();
-  double mu = 0.0, mass = 0.0;
-  if (sub == 0 && live) {
-    double tp = 0, ep = 0, tt = 0, et = 0;
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      nsum<kComp>(tp, ep, s_part[i][0][lane]);
-      nsum<kComp>(tt, et, s_part[i][1][lane]);
-    }
-    node_result(a, k, n, ux, uy, tp - ep, tt - et, mu, mass);
+  for (int o = N; o < 64; o *= 2) {
+    bp += __shfl_xor(bp, o, 64);
+    bt += __shfl_xor(bt, o, 64);
   }
-  // Only the first wavefront holds results.  In a step the block that is
-  // last to leave its partials runs the epilogue (its own launch took 6 us
-  // of a 54 us step at 5,763 triangles x 128): each block's are past the
-  // caches before it counts itself, and on GETMAC's steps, where the epilogue
-  // reads every node field, those are too.
-  const bool last = a.fin.record >= 0;
-  const bool gather = last && gather_step(a.fin.scal[6]);
-  if (sub == 0) {
-    for (int o = 32; o > 0; o >>= 1) {
+  __syncthreads();  // every wavefront has read the first sums
+  if (lane < N) {
+    s_part[wave][0][node] = bp;
+    s_part[wave][1][node] = bt;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    double mu = 0.0, mass = 0.0;
+    if (lane < N && live) {
+      double tp = 0, ep = 0, tt = 0, et = 0;
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        nsum<kComp>(tp, ep, s_part[i][0][node]);
+        nsum<kComp>(tt, et, s_part[i][1][node]);
+      }
+      node_result(a, k, n, ux, uy, tp - ep, tt - et, mu, mass);
+    }
+#pragma unroll
+    for (int o = N / 2; o > 0; o >>= 1) {
       mu = fmax(mu, __shfl_down(mu, o, 64));
       mass += __shfl_down(mass, o, 64);
     }
     if (lane == 0) {
-      agent_store(a.mu_part + blockIdx.x, mu);
-      agent_store(a.mass_part + blockIdx.x, mass);
-    }
-    if (last) {
-      if (gather) __threadfence();
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (lane == 0)
-        s_last = __hip_atomic_fetch_add(a.fin.count, 1, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+      a.mu_part[blockIdx.x] = mu;
+      a.mass_part[blockIdx.x] = mass;
     }
   }
-  if (!last) return;
-  __syncthreads();
-  if (!s_last) return;
-  if (gather) __threadfence();
-  final_body(a.fin, s_red);
-  if (threadIdx.x == 0) *a.fin.count = 0;  // for the next launch
 }
 
 __global__ void __launch_bounds__(256) k_points(const double* __restrict__ mom,
@@ -1697,7 +1767,6 @@ struct Ctx {
          *pts = nullptr, *ps_glob = nullptr, *coord = nullptr, *res_part = nullptr,
          *mu_part = nullptr, *mass_part = nullptr, *scal = nullptr, *ps4 = nullptr,
          *msum = nullptr;
-  int* count = nullptr;     // moments blocks done in this launch
   float* ephase = nullptr;  // [E] FP32 store dither phase per element
   StepRec* rec = nullptr;
   int rec_cap = 0;
@@ -1708,6 +1777,7 @@ struct Ctx {
   int dither = 1;    // FP32 bulk: unbiased (dithered) rounding of the f store
   int mom_split = 1; // moments kernel: wavefronts per node
   int mom_once = 0;  // k_moments_once
+  int mom_lanes = 1; // its lanes per node, L
   int ntiles = 0, vchunk = 1, nvchunks = 1, nblk_upd = 0, nblk_wall = 0, ngroups = 1,
       nblk_mom = 0, neta = 0, nforce = 0;
   int itime = 0;
@@ -1727,23 +1797,36 @@ struct Ctx {
 
 namespace {
 
-FinalArgs final_args(const Ctx& c, int record) {
+// ahead: steps of the batch before this one (k_moments_once; 0 elsewhere)
+FinalArgs final_args(const Ctx& c, int record, int ahead) {
   FinalArgs a;
-  a.res_part = c.res_part; a.nres = c.nblk_upd + c.nblk_wall;
+  a.nres = c.nblk_upd + c.nblk_wall;
+  a.res_part = c.res_part + (ahead & 1 ? 2 * (size_t)a.nres : 0);
   a.mu_part = c.mu_part; a.mass_part = c.mass_part; a.nmom = c.nblk_mom;
   a.fside = c.fside; a.nf = c.nforce; a.coord = c.coord; a.ps_glob = c.ps_glob;
   a.scal = c.scal; a.rec = c.rec; a.rec_cap = c.rec_cap; a.record = record;
   a.mom = c.mom; a.rj = c.rj; a.ptr = c.pt_ptr; a.node = c.pt_node; a.pts = c.pts;
   a.E = c.p.E; a.P = c.p.P; a.mm = c.p.prm.m / kNa; a.rgas = c.p.prm.rgas;
-  a.count = c.count;
+  a.ahead = ahead; a.end = 1;
   return a;
 }
 
+template <typename T, int S>
+void launch_once(Ctx& c, const MomArgs<T>& m) {
+  const dim3 g(c.nblk_mom), b(64 * S);
+  if constexpr (sizeof(T) == 8) {
+    if (c.mom_lanes == 4) {
+      hipLaunchKernelGGL((k_moments_once<T, S, 4>), g, b, 0, c.stream, m);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_moments_once<T, S, 1>), g, b, 0, c.stream, m);
+}
+
 // sums: the kernel that wrote f left its first-pass sums in msum (if it
-// leaves any: fuse_mom); in_step: k_moments_once also runs the step's
-// epilogue
+// leaves any: fuse_mom)
 template <typename T>
-int launch_moments(Ctx& c, bool sums, bool in_step) {
+int launch_moments(Ctx& c, bool sums) {
   MomArgs<T> m;
   m.f = (const T*)c.f[c.cur];
   m.vtd = c.vtd;
@@ -1762,14 +1845,10 @@ int launch_moments(Ctx& c, bool sums, bool in_step) {
   m.E = c.p.E;
   m.ldf = (long long)c.ldf;
   m.V = c.p.V;
-  m.fin = final_args(c, c.mom_once && in_step ? 0 : -1);
   const dim3 g(c.nblk_mom);
-  if (c.mom_once && c.mom_split == 4)
-    hipLaunchKernelGGL((k_moments_once<T, 4>), g, dim3(256), 0, c.stream, m);
-  else if (c.mom_once && c.mom_split == 8)
-    hipLaunchKernelGGL((k_moments_once<T, 8>), g, dim3(512), 0, c.stream, m);
-  else if (c.mom_once)
-    hipLaunchKernelGGL((k_moments_once<T, 16>), g, dim3(1024), 0, c.stream, m);
+  if (c.mom_once && c.mom_split == 4) launch_once<T, 4>(c, m);
+  else if (c.mom_once && c.mom_split == 8) launch_once<T, 8>(c, m);
+  else if (c.mom_once) launch_once<T, 16>(c, m);
   else if (c.mom_split == 8)
     hipLaunchKernelGGL((k_moments<T, 8>), g, dim3(512), 0, c.stream, m);
   else if (c.mom_split == 4)
@@ -1782,8 +1861,11 @@ int launch_moments(Ctx& c, bool sums, bool in_step) {
   return kOk;
 }
 
-int launch_final(Ctx& c, int record) {
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(1024), 0, c.stream, final_args(c, record));
+int launch_final(Ctx& c, int record, int ahead = 0) {
+  // the block of the update's epilogue where that takes a batch's other
+  // steps, so that all sum in one order
+  const dim3 b(c.mom_once && record >= 0 ? c.slots : 1024);
+  hipLaunchKernelGGL(k_final, dim3(1), b, 0, c.stream, final_args(c, record, ahead));
   HIPCK(hipGetLastError());
   return kOk;
 }
@@ -1835,7 +1917,7 @@ void tend(Ctx& c, int k) {
 
 template <typename T, int kS>
 void launch_update_s(Ctx& c, const UpdArgs<T>& u) {
-  const dim3 g(c.neta + c.nblk_upd), b(kS);
+  const dim3 g(c.neta + u.pending + c.nblk_upd), b(kS);
   if (u.cmminc) {  // IMMAT = 0 runs at prefetch depth 1 (set at create)
     if (c.fuse_mom)
       hipLaunchKernelGGL((k_update<T, 1, true, kS, true>), g, b, 0, c.stream, u);
@@ -1891,7 +1973,7 @@ void launch_update(Ctx& c, const UpdArgs<T>& u) {
 }
 
 template <typename T>
-int step_once(Ctx& c) {
+int step_once(Ctx& c, int j, int n) {
   const Prep& p = c.p;
   const T* fc = (const T*)c.f[c.cur];
   T* fn = (T*)c.f[1 - c.cur];
@@ -1901,7 +1983,15 @@ int step_once(Ctx& c) {
   u.emask = c.emask; u.ewslot = c.ewslot; u.np = (const T*)c.np; u.vrow = (const T*)c.vrow;
   u.tiles = c.tiles; u.halo = c.halo; u.wpart = (T*)c.wpart; u.msum = c.msum;
   u.vtd = c.vtd; u.eta_side = c.eta_side; u.eta_geo = c.eta_geo; u.eta = c.eta; u.neta = c.neta;
-  u.scal = c.scal; u.res_part = c.res_part; u.res_stride = c.nblk_upd + c.nblk_wall;
+  // k_moments_once's steps: the epilogue of all but a batch's last goes with
+  // the next step's update, which writes the other half of res_part
+  const bool carry = c.mom_once;
+  double* const res = c.res_part + (carry && (j & 1) ? 2 * (size_t)(c.nblk_upd + c.nblk_wall) : 0);
+  u.fin = final_args(c, 0, j - 1);
+  u.fin.end = 0;
+  u.pending = carry && j > 0;
+  u.ahead = carry ? j : 0;
+  u.scal = c.scal; u.res_part = res; u.res_stride = c.nblk_upd + c.nblk_wall;
   u.E = p.E; u.V = p.V; u.ntiles = c.ntiles; u.vchunk = c.vchunk;
   u.ephase = c.ephase;
   u.ldf = (long long)c.ldf;
@@ -1919,7 +2009,8 @@ int step_once(Ctx& c) {
     w.refl_t = (const T*)c.refl_t; w.wall_bside = c.wall_bside; w.eta = c.eta;
     w.wall_elems = c.wall_elems; w.wpart = (const T*)c.wpart; w.scal = c.scal;
     w.ephase = c.ephase;
-    w.res_part = c.res_part + c.nblk_upd; w.res_stride = c.nblk_upd + c.nblk_wall;
+    w.ahead = u.ahead;
+    w.res_part = res + c.nblk_upd; w.res_stride = c.nblk_upd + c.nblk_wall;
     w.alpha = (T)p.prm.alpha; w.E = p.E; w.V = p.V;
     w.ldf = (long long)c.ldf;
     w.dither = c.dither;
@@ -1937,12 +2028,12 @@ int step_once(Ctx& c) {
   }
   c.cur = 1 - c.cur;
   tbegin(c, 2);
-  int st = launch_moments<T>(c, true, true);
+  int st = launch_moments<T>(c, true);
   if (st) return st;
   tend(c, 2);
-  if (c.mom_once) return kOk;
+  if (carry && j + 1 < n) return kOk;
   tbegin(c, 4);
-  st = launch_final(c, 0);  // with GETMAC's point gather every 1000th step
+  st = launch_final(c, 0, carry ? j : 0);  // with GETMAC's point gather every 1000th step
   tend(c, 4);
   return st;
 }
@@ -1957,7 +2048,7 @@ int capture_graph(Ctx& c) {
   if (c.graph_exec[slot]) return kOk;
   HIPCK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
   int st = kOk;
-  for (int s = 0; s < kGraphSteps && st == kOk; ++s) st = step_once<T>(c);
+  for (int s = 0; s < kGraphSteps && st == kOk; ++s) st = step_once<T>(c, s, kGraphSteps);
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(c.stream, &g);
   if (st) {
@@ -1985,8 +2076,8 @@ int run_steps(Ctx& c, int n) {
       done += kGraphSteps;
     }
   }
-  for (; done < n; ++done) {
-    int st = step_once<T>(c);
+  for (int j = 0, m = n - done; j < m; ++j) {
+    int st = step_once<T>(c, j, m);
     if (st) return st;
   }
   return kOk;
@@ -2168,7 +2259,6 @@ int upload_tables(Ctx& c) {
   if ((st = upload(&c.intma, p.intma, c.owned))) return st;
   std::vector<double> eta0(std::max(p.B, 1), 0.0);
   if ((st = upload(&c.eta, eta0, c.owned))) return st;
-  if ((st = upload(&c.count, std::vector<int>{0}, c.owned))) return st;
   if ((st = alloc((T**)&c.np, 5 * N3, c.owned))) return st;
   if ((st = alloc(&c.mom, 5 * N3, c.owned))) return st;
   if ((st = alloc(&c.pts, 6 * (size_t)p.P, c.owned))) return st;
@@ -2205,11 +2295,11 @@ int seed_points(Ctx& c, const std::vector<double>& ps4) {
 // (sums: whoever wrote f left its first-pass sums)
 template <typename T>
 int refresh(Ctx& c, bool sums) {
-  int st = launch_moments<T>(c, sums, false);
+  int st = launch_moments<T>(c, sums);
   if (st) return st;
   if ((st = launch_points(c, 1))) return st;
   // DTE for the next step, no record
-  HIPCK(hipMemsetAsync(c.res_part, 0, 2 * sizeof(double) * (c.nblk_upd + c.nblk_wall), c.stream));
+  HIPCK(hipMemsetAsync(c.res_part, 0, 4 * sizeof(double) * (c.nblk_upd + c.nblk_wall), c.stream));
   return launch_final(c, -1);
 }
 
@@ -2416,6 +2506,12 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   // 19; 5,763 x 512 97 -> 85, 77 -> 52; 10,820 x 512 (8112 wavefronts) 133
   // -> 126, 91 -> 69; 21,178 x 512 (15888) 208 -> 236, 124 -> 121; 41,389 x
   // 512 374 -> 442, 203 -> 228; 41,389 x 128 (7760) 118 -> 115, 71 -> 62.
+  // Four lanes a node in FP64 while 64 nodes a block come to 320 blocks or
+  // fewer, which leave the CUs idle or unevenly loaded.  A step, us, one lane
+  // -> four: 1,500 x 128 23.3 -> 21.5, 2,590 x 128 25.6 -> 24.4, x 256 34.0 ->
+  // 31.9, x 512 50.3 -> 48.3, 5,763 (271 blocks) x 128 35.3 -> 34.3, x 512
+  // 88.4 -> 82.9; 10,820 (508) x 128 45.6 -> 47.5, x 256 71.2 -> 76.2.  FP32
+  // has half the bytes a row: 1,500 x 128 18.9 -> 19.1, 5,763 26.9 -> 29.7.
   // DGBGK_MOM_SPLIT asks for k_moments.
   if (!std::getenv("DGBGK_MOM_SPLIT") && c.p.V <= 16 * kMomHold) {
     const int S = c.p.V <= 4 * kMomHold ? 4 : (c.p.V <= 8 * kMomHold ? 8 : 16);
@@ -2423,6 +2519,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
     if (waves <= (c.prec ? 16384 : 8192)) {
       c.mom_once = 1;
       c.mom_split = S;
+      c.mom_lanes = !c.prec && waves / S <= 320 ? 4 : 1;
       c.fuse_mom = 0;
     }
   }
@@ -2513,7 +2610,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
       const int v = std::atoi(ms);
       if (v == 1 || v == 2 || v == 4 || v == 8) c.mom_split = v;
     }
-    const size_t per = c.mom_once ? 64 : std::max(64, 256 / c.mom_split);
+    const size_t per = c.mom_once ? 64 / c.mom_lanes : std::max(64, 256 / c.mom_split);
     c.nblk_mom = (int)((n3 + per - 1) / per);
   }
   c.neta = (int)p.eta_side.size();
@@ -2521,7 +2618,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   st = c.prec ? upload_tables<float>(c) : upload_tables<double>(c);
   if (st) return cleanup(st);
   if (!c.eorder.empty() && (st = upload(&c.d_eorder, c.eorder, c.owned))) return cleanup(st);
-  if ((st = alloc(&c.res_part, 2 * ((size_t)c.nblk_upd + c.nblk_wall), c.owned)))
+  if ((st = alloc(&c.res_part, 4 * ((size_t)c.nblk_upd + c.nblk_wall), c.owned)))
     return cleanup(st);
   if ((st = alloc(&c.msum, (size_t)c.nvchunks * 3 * 3 * (size_t)p.E, c.owned)))
     return cleanup(st);

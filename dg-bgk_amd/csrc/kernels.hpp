@@ -47,6 +47,29 @@ constexpr int kUpdOwn = 1 << 5;    // boundary side: the own element's values
 constexpr int kUpdInflow = 1 << 6; // inflow side: upwind values are zero (FP32 form)
 constexpr int kUpdSlot = 8;     // bits 8+: neighbour's LDS slot
 
+// The step's epilogue (k_final, or a block of the next step's k_update).
+struct FinalArgs {
+  const double* res_part;  // [2][nres] of the update and wall passes
+  const double* mu_part;   // [nmom] of the moments blocks
+  const double* mass_part;
+  const int* fside;        // [nf][2] points of the force sides
+  const double* coord;
+  double* ps_glob;
+  double* scal;
+  StepRec* rec;
+  const double* mom;       // GETMAC's point gather, on every 1000th step
+  const double* rj;
+  const int* ptr;
+  const int* node;
+  double* pts;
+  int nres, nmom, nf, rec_cap;
+  int record;              // < 0: outside a step
+  int ahead;               // this step's place in its batch (scal[6]: as it began)
+  int end;                 // scal[6] moves on to this step
+  int E, P;
+  double mm, rgas;
+};
+
 template <typename T>
 struct UpdArgs {
   const T* __restrict__ fcur;
@@ -76,6 +99,9 @@ struct UpdArgs {
   long long ldf;  // row stride of f
   int dither;     // FP32: dithered (unbiased) rounding of the f store
   int cmminc;     // IMMAT = 0: CMMINC's increment and residual (geo row 7 its row sum)
+  FinalArgs fin;  // the step before: its epilogue if pending
+  int pending;
+  int ahead;      // this step's place in its batch
 };
 
 template <typename T>
@@ -107,28 +133,7 @@ struct WallArgs {
   long long ldf;  // row stride of f
   int dither;     // FP32: dithered (unbiased) rounding of the f store
   int cmminc;     // IMMAT = 0: as in UpdArgs
-};
-
-// The step's epilogue (k_final).
-struct FinalArgs {
-  const double* res_part;  // [2][nres] of the update and wall passes
-  const double* mu_part;   // [nmom] of the moments blocks
-  const double* mass_part;
-  const int* fside;        // [nf][2] points of the force sides
-  const double* coord;
-  double* ps_glob;
-  double* scal;
-  StepRec* rec;
-  const double* mom;       // GETMAC's point gather, on every 1000th step
-  const double* rj;
-  const int* ptr;
-  const int* node;
-  double* pts;
-  int* count;              // moments blocks done (k_moments_once)
-  int nres, nmom, nf, rec_cap;
-  int record;              // < 0: outside a step
-  int E, P;
-  double mm, rgas;
+  int ahead;
 };
 
 template <typename T>
@@ -147,7 +152,6 @@ struct MomArgs {
   double mm, sigt;
   int E, V, nchunks, vchunk;
   long long ldf;  // row stride of f
-  FinalArgs fin;  // k_moments_once; record < 0: no epilogue
 };
 
 }  // namespace dgbgk

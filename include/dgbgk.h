@@ -180,7 +180,7 @@ void dgbgk_setup_destroy(dgbgk_setup *s);
 
 /* Kernel timing with HIP events on the context's stream.  Kernel ids:
  * 0 update, 1 wall pass, 2 moments, 3 eta (part of 0: never counted),
- * 4 finalize+forces (part of 2 on small meshes), 5 points. */
+ * 4 finalize+forces (on small meshes once per batch of steps, else part of 0), 5 points. */
 int dgbgk_timing(dgbgk_ctx *ctx, int enable);
 int dgbgk_kernel_time(dgbgk_ctx *ctx, int kernel, double *ms_total, long *count);
 int dgbgk_sync(dgbgk_ctx *ctx);
