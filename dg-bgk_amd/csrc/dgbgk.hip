@@ -250,13 +250,13 @@ template <typename T>
 struct SlotState {
   T gx[3], gy[3], pA[3], pB[3], pU[3], pV[3], pMd[3];  // phase A (all slots)
   T gxa[3], gya[3], mdt, nx[3], ny[3];                 // phase B (owned slots)
-  int mask, wsl, e;
+  unsigned cls;  // upwind choice and inflow nodes (own_upwind)
+  int e;
   // LDS index (4 slot + node) of the neighbour's values at k, k1; a boundary
   // side reads its own element's, an FP32 inflow side the slot of zeros
   int nb1[3], nb2[3];
-  bool inflow[3];      // FP32: the own values are never upwind (a lane mask, in SGPRs)
   float dph;           // FP32 store dither: the element's fixed phase
-  bool owned, active;
+  bool owned, active, wall;
 };
 
 template <typename T>
@@ -272,15 +272,32 @@ __device__ __forceinline__ void store4<double>(double* p, double a, double b, do
   reinterpret_cast<double2*>(p)[1] = make_double2(c, d);
 }
 
+// The upwind choice of the three sides and the inflow nodes in one register
+// (SlotState::cls).  Side k's field, from bit kClsSide[k], is the set of
+// v_cmp_class for which the own values are upwind: w negative; w negative or
+// zero on the side's right element, whose values both elements take on a tie;
+// none on an FP32 inflow side.  The instruction reads ten bits, of which 0-2
+// (NaN, -inf) never apply, w being finite: they hold the inflow nodes.  One
+// compare and at most one shift a side: FP32 299 us at 101,753 x 512 (297
+// with w < 0 alone, which lets NaN cross a tie; 309 with a second compare per
+// side), FP64 637 (632, 648).
+constexpr int kClsSide[3] = {0, 16, 25};
+constexpr unsigned kClsNeg = 0x18, kClsZero = 0x60;  // negative, both zeros
+template <typename T>
+__device__ __forceinline__ bool own_upwind(T w, unsigned cls, int k) {
+  if constexpr (sizeof(T) == 8) return __builtin_amdgcn_class(w, cls >> kClsSide[k]);
+  else return __builtin_amdgcn_classf(w, cls >> kClsSide[k]);
+}
+
 // The scalars of one ordinate: a row of vrow, read by scalar loads one
 // ordinate ahead, right after the barrier: a scalar load still in flight at
 // the barrier would be waited for there (one counter for scalar and LDS
 // operations), before every wavefront's second half.  With the row, the
 // upwind select on one compare (no side has a case of its own) and absmax,
 // an element and ordinate takes 116 vector and 39 scalar instructions in
-// FP32 (154 and 77 before) and 137 vector ones in FP64 (172).  FP32 is bound
-// by them: update 325 -> 306 us at 101,753 x 512, 351 -> 326 us at 25,781 x
-// 2048; FP64 by memory: 626 -> 629 us.
+// FP32 (154 and 77 before) and 137 vector ones in FP64 (172), without the
+// tie rule's shifts.  FP32 is bound by them: update 325 -> 306 us at 101,753 x
+// 512, 351 -> 326 us at 26,237 x 2048; FP64 by memory: 626 -> 629 us.
 template <typename T>
 struct OrdRow {
   T ux, uy, fin, ph;   // velocity, inflow value, FP32 store dither phase
@@ -359,11 +376,14 @@ template <typename T, bool kMom, bool kCM>
 __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotState<T>& s,
                                               Half<T>& o, int v, const OrdRow<T>& r, float ph,
                                               float dsc0, float dsc1, bool anyin,
-                                              const T (&f)[3], const T* __restrict__ sf, T& res,
+                                              const T (&f)[3], const T* __restrict__ sf,
+                                              const int* wslot, T& res,
                                               T& chg, double (&m0)[3], double (&m1)[3],
                                               double (&m2)[3]) {
   const T c13 = T(1) / T(3);
   const T ux = r.ux, uy = r.uy, fin = r.fin, U = o.U;
+  unsigned cls = s.cls;
+  asm volatile("" : "+v"(cls));  // its fields are taken here, not kept apart
   T(&cold)[3] = o.cold;
   T(&h)[3] = o.h;
   T rhs[3];
@@ -379,16 +399,17 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
     // M2 = [[2,1],[1,2]] and g = f - U of the upwind element.  The reference
     // orients each side once (left element) and subtracts the left element's
     // flux from the right element; with the right element's outward normal
-    // that is the same expression.  Upwind: own values when c.n > 0; on a
-    // tie the flux is zero whichever element's values it takes; on an outflow
-    // side the neighbour's are the own; inflow and wall sides carry a zero
-    // (len/6) n here.
+    // that is the same expression.  Upwind: own values when c.n > 0, on a
+    // tie the right element's, as in the reference (the flux is then zero if
+    // they are finite, NaN if they are not); on an outflow side the
+    // neighbour's are the own; inflow and wall sides carry a zero (len/6) n
+    // here.
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int k1 = (k + 1) % 3;
       // w = -(len/6) c.n from the edge's (len/6) n: c.n > 0 exactly when w < 0
       const T w = -(ux * s.nx[k] + uy * s.ny[k]);
-      const bool own = w < T(0);
+      const bool own = own_upwind(w, cls, k);
       // the neighbour's values are read whichever side is upwind (fixed LDS
       // indices, no address arithmetic); the element's own are in registers
       const T n1 = sf[s.nb1[k]], n2 = sf[s.nb2[k]];
@@ -411,7 +432,7 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
     for (int k = 0; k < 3; ++k) {
       const int k1 = (k + 1) % 3;
       const T w = -(ux * s.nx[k] + uy * s.ny[k]);
-      const bool own = w < T(0) && !s.inflow[k];
+      const bool own = own_upwind(w, cls, k);
       const T n1 = sf[s.nb1[k]], n2 = sf[s.nb2[k]], un = sf[s.nb1[k] | 3];
       const T du = un - U;
       T e1 = ((n1 - f[0]) - db) - du, e2 = ((n2 - f[0]) - db) - du;
@@ -424,8 +445,8 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
       rhs[k1] += w * (g1 + T(2) * g2);
     }
   }
-  if (s.wsl >= 0) {
-    T* wp = a.wpart + ((size_t)s.wsl * a.V + v) * 8;
+  if (s.wall) {
+    T* wp = a.wpart + ((size_t)wslot[threadIdx.x] * a.V + v) * 8;
     store4(wp, rhs[0], rhs[1], rhs[2], cold[0]);
     store4(wp + 4, cold[1], cold[2], U, T(0));
     return;
@@ -459,7 +480,7 @@ __device__ __forceinline__ void update_second(const UpdArgs<T>& a, const SlotSta
   if (anyin) {  // inflow nodes: rare; a wave-uniform branch
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      if ((s.mask >> k) & 1) {
+      if ((cls >> k) & 1) {
         fn[k] = fin;
         if constexpr (sizeof(T) == 4) cg[k] = fabs(fin - f[k]);
       }
@@ -708,6 +729,7 @@ k_update(UpdArgs<T> a) {
   __shared__ __align__(16) T s_f[kQ][kRow];
   if (sizeof(T) == 4 && threadIdx.x < 4 * kQ)  // read after the first barrier
     s_f[threadIdx.x / 4][kS * 4 + threadIdx.x % 4] = T(0);
+  __shared__ int s_wsl[kS];  // wall slots: a register less than kept apart
   __shared__ double s_red[6][16];
   if ((int)blockIdx.x < a.neta) {
     wall_eta(a, blockIdx.x, s_red[0]);
@@ -765,15 +787,14 @@ k_update(UpdArgs<T> a) {
   for (int k = 0; k < 3; ++k) {
     s.gx[k] = s.gy[k] = s.pA[k] = s.pB[k] = s.pU[k] = s.pV[k] = s.pMd[k] = T(0);
     s.gxa[k] = s.gya[k] = s.nx[k] = s.ny[k] = T(0);
-    s.inflow[k] = false;
     s.nb1[k] = 4 * slot + k;
     s.nb2[k] = 4 * slot + (k + 1) % 3;
 
   }
   s.mdt = T(0);
   s.dph = 0.f;
-  s.mask = 0;
-  s.wsl = -1;
+  s.cls = 0;
+  s.wall = false;
   if (s.active) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -790,8 +811,10 @@ k_update(UpdArgs<T> a) {
   if (s.owned) {
     const T area = a.geo[6 * E + e];
     s.mdt = a.geo[7 * E + e] * dte;
+    s.cls = a.emask[e];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
+      s.cls |= kClsNeg << kClsSide[k];
       s.gxa[k] = s.gx[k] * area;
       s.gya[k] = s.gy[k] * area;
       const int in = a.uinfo[k * E + e];
@@ -799,15 +822,17 @@ k_update(UpdArgs<T> a) {
         const int nbs = in >> kUpdSlot;
         s.nb1[k] = 4 * nbs + ((in >> kUpdNbK) & 3);
         s.nb2[k] = 4 * nbs + ((in >> kUpdNbK1) & 3);
+        if (in & kUpdRight) s.cls |= kClsZero << kClsSide[k];
       } else if (sizeof(T) == 4 && (in & kUpdInflow)) {
         s.nb1[k] = s.nb2[k] = 4 * kS;
-        s.inflow[k] = true;
+        s.cls &= ~(kClsNeg << kClsSide[k]);
       }
       s.nx[k] = a.unx[k * E + e];
       s.ny[k] = a.uny[k * E + e];
     }
-    s.mask = a.emask[e];
-    s.wsl = a.ewslot[e];
+    const int ws = a.ewslot[e];
+    s.wall = ws >= 0;
+    s_wsl[slot] = ws;  // read by this thread only
     s.dph = a.ephase[e];
   }
   T res = 0, chg = 0;
@@ -815,7 +840,7 @@ k_update(UpdArgs<T> a) {
   const double stw = (a.scal[6] + a.ahead) * 0.6180339887498949;  // Weyl step phase
   const float sph = (float)(stw - floor(stw));
   const float dsc0 = a.dither ? 0x1p-23f : 0.f, dsc1 = a.dither ? -0x1p-24f : 0.f;
-  const bool anyin = __ballot(s.mask != 0) != 0;
+  const bool anyin = __ballot((s.cls & 7) != 0) != 0;
   const T* fe = a.fcur + 3 * (size_t)e;
   // prime the queue: f of v0 .. v0+kDepth-1, and the first ordinate's row
   T q[kQ][3];
@@ -849,11 +874,11 @@ k_update(UpdArgs<T> a) {
         row = ord_row<T, kMom>(a.vrow, min(v + 1, v1 - 1));
         if (s.owned)
           update_second<T, kMom, kCM>(a, s, hf, v, cur, sph + (float)cur.ph, dsc0, dsc1, anyin,
-                                      q[j], s_f[j], res, chg, m0, m1, m2);
+                                      q[j], s_f[j], s_wsl, res, chg, m0, m1, m2);
       }
     }
   }
-  if (kMom && s.owned && s.wsl < 0) {
+  if (kMom && s.owned && !s.wall) {
     double* ms = a.msum + (size_t)(logical / a.ntiles) * 3 * N3 + 3 * (size_t)e;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -2155,7 +2180,7 @@ int upload_tables(Ctx& c) {
       uny[i] = flux ? (T)(sg * ed.alen * ed.ny) : T(0);
       if (ed.kind == kInterior) {
         const int nbk = ed.sign > 0 ? ed.b1 : ed.b2, nbk1 = ed.sign > 0 ? ed.b2 : ed.b1;
-        uinfo[i] = (nbk << kUpdNbK) | (nbk1 << kUpdNbK1) |
+        uinfo[i] = (nbk << kUpdNbK) | (nbk1 << kUpdNbK1) | (ed.sign > 0 ? 0 : kUpdRight) |
                    (p.nbr_slot[3 * (size_t)e + k] << kUpdSlot);
       } else {
         uinfo[i] = kUpdOwn | (ed.kind == kInflow ? kUpdInflow : 0);

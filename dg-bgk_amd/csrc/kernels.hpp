@@ -40,9 +40,11 @@ struct StepRec {  // same layout as dgbgk_step_info
 };
 
 // Update-kernel edge word (uinfo), one per element edge k (local nodes k,
-// k1 = (k+1)%3): the flux source when the neighbour is upwind.
+// k1 = (k+1)%3): the flux source when the neighbour is upwind and the tie
+// rule of the side's orientation.
 constexpr int kUpdNbK = 0;      // bits 0-1: neighbour's local node at node k
 constexpr int kUpdNbK1 = 2;     // bits 2-3: neighbour's local node at node k1
+constexpr int kUpdRight = 1 << 4;  // this element is the side's right element
 constexpr int kUpdOwn = 1 << 5;    // boundary side: the own element's values
 constexpr int kUpdInflow = 1 << 6; // inflow side: upwind values are zero (FP32 form)
 constexpr int kUpdSlot = 8;     // bits 8+: neighbour's LDS slot
