@@ -1613,7 +1613,11 @@ __global__ void __launch_bounds__(256) k_seed(T* __restrict__ f, const int* __re
   T* o = f + (size_t)vb * ldf + k;
   for (int v = vb; v < ve; ++v, o += ldf) {
     const double dx = ldc(vtd, 2 * V + v) - u0, dy = ldc(vtd, 3 * V + v) - v0;
-    const T x = (T)(n1 * (c0 * mexp(-(b2 * (dx * dx + dy * dy)))));
+    // mexp's reduction leaves its interval from about -1e16 on and is NaN at
+    // -inf; below -800 the exponential is 0 (the caller's state may be cold
+    // or fast without bound, and NaN stays NaN)
+    const double ex = -(b2 * (dx * dx + dy * dy));
+    const T x = (T)(n1 * (c0 * mexp(ex < -800.0 ? -800.0 : ex)));
     fstore_nt(o, x);
     if (kMom) {
       m0 = fma(ldc(vtd, 4 * V + v), (double)x, m0);
