@@ -1432,6 +1432,9 @@ __global__ void __launch_bounds__(S > 4 ? 64 * S : 256) k_moments(MomArgs<T> a) 
 // and a quarter of the serial work, and the tables, whose rows then differ
 // between lanes, come from LDS.  A block's second pass alone took 4 of the 17
 // us at 5,763 x 128 with one wavefront per SIMD.
+// The FP32 pairs take 0.7 us of 9.6 at 1,679 x 128 and 3 of 31 at 5,763 x 512,
+// and keep the density's error at its own rounding (7.5e-17 RMS; plain sums of
+// a wavefront's 32 ordinates 1.5e-16).
 // Nothing follows the blocks' partial results: that its last block ran the
 // step's epilogue cost 10 ns a block in counting them and 4 us of loads and
 // reductions behind them (5,763 x 128, a step: 38.6 us, 35.3 without).
@@ -1477,8 +1480,10 @@ k_moments_once(MomArgs<T> a) {
       if (i == 3 || i == 4) return (double)ldc(a.vtab + (i - 3) * V + vb, j);
     return ldc(a.vtd + (i < 3 ? 4 + i : (kComp ? 7 : i - 3)) * V + vb, j);
   };
-  // the share's ordinates; scalar loads in runs of four, then one by one
-  auto each = [&](auto&& body) {
+  // the share's ordinates; L = 1: scalar loads in runs of four, then one by
+  // one, and at each run's end fold(): FP32 sums are pairs (sum, correction),
+  // as in k_moments
+  auto each = [&](auto&& body, auto&& fold) {
     if constexpr (L > 1) {
 #pragma unroll
       for (int j = 0; j < H; ++j)
@@ -1489,21 +1494,46 @@ k_moments_once(MomArgs<T> a) {
         if (j + 4 <= cnt) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) body(j + i);
-        } else {
+          fold();
+        } else if (j < cnt) {
 #pragma unroll
           for (int i = 0; i < 3; ++i)
             if (j + i < cnt) body(j + i);
+          fold();
         }
       }
     }
   };
-  double b0 = 0, b1 = 0, b2 = 0;
-  each([&](int j) {
-    const double fd = (double)f[j];
-    b0 = fma(tab(0, j), fd, b0);
-    b1 = fma(tab(1, j), fd, b1);
-    b2 = fma(tab(2, j), fd, b2);
-  });
+  auto add = [](double& s, double& c, double& b) {  // a run's sum into its pair
+    if (kComp) {
+      nsum<true>(s, c, b);
+      b = 0.0;
+    }
+  };
+  double b0 = 0, b1 = 0, b2 = 0, s0 = 0, c0 = 0, s1 = 0, c1 = 0, s2 = 0, c2 = 0;
+  each(
+      [&](int j) {
+        const double fd = (double)f[j];
+        b0 = fma(tab(0, j), fd, b0);
+        b1 = fma(tab(1, j), fd, b1);
+        b2 = fma(tab(2, j), fd, b2);
+        if (j & 1) {  // the momenta cancel: in runs of two
+          add(s1, c1, b1);
+          add(s2, c2, b2);
+        }
+      },
+      [&] {
+        add(s0, c0, b0);
+        if (cnt & 1) {
+          add(s1, c1, b1);
+          add(s2, c2, b2);
+        }
+      });
+  if (kComp) {
+    b0 = s0 - c0;
+    b1 = s1 - c1;
+    b2 = s2 - c2;
+  }
 #pragma unroll
   for (int o = N; o < 64; o *= 2) {
     b0 += __shfl_xor(b0, o, 64);
@@ -1527,21 +1557,30 @@ k_moments_once(MomArgs<T> a) {
   const bool dens = n >= 1e-20;
   const double ux = dens ? (t1 - e1) / n : 0.0, uy = dens ? (t2 - e2) / n : 0.0;
   const float uxf = (float)ux, uyf = (float)uy;
-  double bp = 0, bt = 0;  // the terms of k_moments' second pass
-  each([&](int j) {
-    if constexpr (kComp) {
-      const float ex = uxf - (float)tab(3, j), ey = uyf - (float)tab(4, j);
-      const float rel = __builtin_amdgcn_sqrtf(fmaf(ex, ex, ey * ey));
-      bp = fma((double)f[j], tab(5, j), bp);
-      bt = fma((double)(rel * (float)f[j]), tab(0, j), bt);
-    } else {
-      const double fw = (double)f[j] * tab(0, j);
-      const double dx = tab(5, j) - ux, dy = tab(6, j) - uy;
-      const double ex = ux - tab(3, j), ey = uy - tab(4, j);
-      bp += 0.5 * (dx * dx + dy * dy) * fw;
-      bt += sqrt(ex * ex + ey * ey) * fw;
-    }
-  });
+  double bp = 0, bt = 0, sp = 0, cp = 0, st = 0, ct = 0;  // k_moments' second pass
+  each(
+      [&](int j) {
+        if constexpr (kComp) {
+          const float ex = uxf - (float)tab(3, j), ey = uyf - (float)tab(4, j);
+          const float rel = __builtin_amdgcn_sqrtf(fmaf(ex, ex, ey * ey));
+          bp = fma((double)f[j], tab(5, j), bp);
+          bt = fma((double)(rel * (float)f[j]), tab(0, j), bt);
+        } else {
+          const double fw = (double)f[j] * tab(0, j);
+          const double dx = tab(5, j) - ux, dy = tab(6, j) - uy;
+          const double ex = ux - tab(3, j), ey = uy - tab(4, j);
+          bp += 0.5 * (dx * dx + dy * dy) * fw;
+          bt += sqrt(ex * ex + ey * ey) * fw;
+        }
+      },
+      [&] {
+        add(sp, cp, bp);
+        add(st, ct, bt);
+      });
+  if (kComp) {
+    bp = sp - cp;
+    bt = st - ct;
+  }
 #pragma unroll
   for (int o = N; o < 64; o *= 2) {
     bp += __shfl_xor(bp, o, 64);
@@ -2530,22 +2569,26 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   // Moments by k_moments_once (and no sums in the update) while its blocks
   // of S wavefronts come in about two rounds of the chip or fewer: S the
   // fewest that hold V ordinates, at most 8192 wavefronts in FP64 and 16384
-  // in FP32 (half the registers, so twice the blocks resident).  Update plus
-  // moments, us, with sums -> without: 1,679 x 128 FP64 41 -> 22, FP32 38 ->
-  // 19; 5,763 x 512 97 -> 85, 77 -> 52; 10,820 x 512 (8112 wavefronts) 133
-  // -> 126, 91 -> 69; 21,178 x 512 (15888) 208 -> 236, 124 -> 121; 41,389 x
-  // 512 374 -> 442, 203 -> 228; 41,389 x 128 (7760) 118 -> 115, 71 -> 62.
+  // in FP32 (half the registers, so twice the blocks resident), where
+  // blocks of 16, one to a CU, stop at 12288.  FP64, update plus moments, us,
+  // with sums -> without: 1,679 x 128 41 -> 22; 5,763 x 512 97 -> 85; 10,820 x
+  // 512 (8112 wavefronts) 133 -> 126; 21,178 x 512 (15888) 208 -> 236; 41,389
+  // x 128 (7760) 118 -> 115.  FP32, a step: 1,679 x 128 43 -> 20; 5,763 x 512
+  // 81 -> 59; 14,949 x 512 (11216) 116 -> 101; 18,129 x 512 (13600) 120 ->
+  // 122; 21,178 x 512 129 -> 133; 41,389 x 128 76 -> 68, x 256 (15528) 117 ->
+  // 118; 81,784 x 128 (15336) 116 -> 107.
   // Four lanes a node in FP64 while 64 nodes a block come to 320 blocks or
   // fewer, which leave the CUs idle or unevenly loaded.  A step, us, one lane
   // -> four: 1,500 x 128 23.3 -> 21.5, 2,590 x 128 25.6 -> 24.4, x 256 34.0 ->
   // 31.9, x 512 50.3 -> 48.3, 5,763 (271 blocks) x 128 35.3 -> 34.3, x 512
   // 88.4 -> 82.9; 10,820 (508) x 128 45.6 -> 47.5, x 256 71.2 -> 76.2.  FP32
-  // has half the bytes a row: 1,500 x 128 18.9 -> 19.1, 5,763 26.9 -> 29.7.
+  // has half the bytes a row: 1,500 x 128 18.9 -> 19.1, 5,763 26.9 -> 29.7
+  // (plain sums).
   // DGBGK_MOM_SPLIT asks for k_moments.
   if (!std::getenv("DGBGK_MOM_SPLIT") && c.p.V <= 16 * kMomHold) {
     const int S = c.p.V <= 4 * kMomHold ? 4 : (c.p.V <= 8 * kMomHold ? 8 : 16);
     const size_t waves = (3 * (size_t)c.p.E + 63) / 64 * S;
-    if (waves <= (c.prec ? 16384 : 8192)) {
+    if (waves <= (!c.prec ? 8192 : S < 16 ? 16384 : 12288)) {
       c.mom_once = 1;
       c.mom_split = S;
       c.mom_lanes = !c.prec && waves / S <= 320 ? 4 : 1;
