@@ -2755,16 +2755,10 @@ int dgbgk_step(dgbgk_ctx* h, int nsteps, dgbgk_step_info* info) {
     c.itime += batch;
     if (info) {
       static_assert(1024 * sizeof(StepRec) <= kStageBlock, "a batch's records fit a block");
-      StageBlock b;
-      char* to = b.p ? b.p : (char*)(info + done);
       const int n1 = std::min(batch, c.rec_cap - first);
-      HIPCK(hipMemcpyAsync(to, c.rec + first, n1 * sizeof(StepRec), hipMemcpyDeviceToHost,
-                           c.stream));
-      if (batch > n1)
-        HIPCK(hipMemcpyAsync(to + n1 * sizeof(StepRec), c.rec, (batch - n1) * sizeof(StepRec),
-                             hipMemcpyDeviceToHost, c.stream));
-      HIPCK(hipStreamSynchronize(c.stream));
-      if (b.p) std::memcpy((void*)(info + done), b.p, batch * sizeof(StepRec));
+      const StagePart rec[2] = {{c.rec + first, info + done, n1 * sizeof(StepRec)},
+                                {c.rec, info + done + n1, (batch - n1) * sizeof(StepRec)}};
+      HIPCK(stage_fetch(rec, batch > n1 ? 2 : 1, c.stream));
     } else {
       HIPCK(hipStreamSynchronize(c.stream));
     }
@@ -2844,14 +2838,10 @@ int dgbgk_point_fields(dgbgk_ctx* h, double* nd, double* rho, double* uvel, doub
   while (i1 > i0 && !dst[i1 - 1]) --i1;
   const size_t row = P * sizeof(double);
   if ((i1 - i0) * row <= kStageBlock) {  // all in one copy
-    StageBlock b;
-    if (b.p) {
-      HIPCK(hipMemcpyAsync(b.p, c.pts + i0 * P, (i1 - i0) * row, hipMemcpyDeviceToHost, c.stream));
-      HIPCK(hipStreamSynchronize(c.stream));
-      for (int i = i0; i < i1; ++i)
-        if (dst[i]) std::memcpy(dst[i], b.p + (i - i0) * row, row);
-      return kOk;
-    }
+    StagePart part[6];
+    for (int i = i0; i < i1; ++i) part[i] = {c.pts + i * P, dst[i], row};
+    HIPCK(stage_fetch(part + i0, i1 - i0, c.stream));
+    return kOk;
   }
   for (int i = i0; i < i1; ++i)
     if (dst[i]) HIPCK(stage_copy(c.pts + i * P, dst[i], row, false, c.stream, c.dev));

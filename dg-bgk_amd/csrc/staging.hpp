@@ -74,13 +74,32 @@ class StagePool {
   int users_ = 0;
 };
 
-// A pinned block for the scope (null if none could be had).
-struct StageBlock {
-  char* p;
-  StageBlock() : p(StagePool::get().take()) {}
-  ~StageBlock() { StagePool::get().give(p); }
+// A pinned block for the scope (p null if none could be had), with the copies
+// a stream carries to or from it.  It goes back idle on every way out of the
+// scope: one that a copy may still use, and whose stream cannot be waited
+// for, is not handed out again.
+class StageBlock {
+ public:
+  char* const p;
+  explicit StageBlock(hipStream_t s) : p(StagePool::get().take()), s_(s) {}
+  ~StageBlock() {
+    if (!busy_ || hipStreamSynchronize(s_) == hipSuccess) StagePool::get().give(p);
+  }
   StageBlock(const StageBlock&) = delete;
   StageBlock& operator=(const StageBlock&) = delete;
+  hipError_t copy(void* to, const void* from, size_t n, hipMemcpyKind kind) {
+    busy_ = true;
+    return hipMemcpyAsync(to, from, n, kind, s_);
+  }
+  hipError_t wait() {
+    const hipError_t e = hipStreamSynchronize(s_);
+    busy_ = busy_ && e != hipSuccess;
+    return e;
+  }
+
+ private:
+  const hipStream_t s_;
+  bool busy_ = false;
 };
 
 // fn(w) for w < n (at most kWorkers), on this thread and n - 1 others that
@@ -102,6 +121,37 @@ void on_workers(int n, int dev, F fn) {
     if (x.joinable()) x.join();
 }
 
+// Small results: device ranges to as many arrays of the caller's (host null:
+// not wanted), at most a block in all, adjacent ranges as one copy.  In order
+// after the work on the stream; the data has arrived, and nothing writes to
+// the arrays any more, on return.
+struct StagePart {
+  const void* dev;
+  void* host;
+  size_t n;
+};
+inline hipError_t stage_fetch(const StagePart* part, int parts, hipStream_t stream) {
+  StageBlock b(stream);
+  hipError_t e = hipSuccess;
+  size_t at = 0;
+  for (int i = 0, j; i < parts && e == hipSuccess; i = j) {
+    size_t n = part[i].n;
+    for (j = i + 1; b.p && j < parts && part[j].dev == (const char*)part[i].dev + n; ++j)
+      n += part[j].n;
+    if (b.p)
+      e = b.copy(b.p + at, part[i].dev, n, hipMemcpyDeviceToHost);
+    else if (part[i].host)
+      e = b.copy(part[i].host, part[i].dev, n, hipMemcpyDeviceToHost);
+    at += n;
+  }
+  const hipError_t f = b.wait();
+  if (e == hipSuccess) e = f;
+  at = 0;
+  for (int i = 0; e == hipSuccess && b.p && i < parts; at += part[i++].n)
+    if (part[i].host) std::memcpy(part[i].host, b.p + at, part[i].n);
+  return e;
+}
+
 // Copies n bytes between the caller's array and device memory, in order
 // after the work on the stream, and returns when the data has arrived.
 // toDev: host is read, else written.
@@ -115,10 +165,11 @@ inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStr
   const size_t pieces = (n + kStageBlock - 1) / kStageBlock;
   if (!n) return hipSuccess;
   if (pieces == 1) {
-    StageBlock b;
+    StageBlock b(stream);
     if (!b.p) return plain((char*)dev, (char*)host, n);
     if (toDev) std::memcpy(b.p, host, n);
-    const hipError_t e = plain((char*)dev, b.p, n);
+    hipError_t e = toDev ? b.copy(dev, b.p, n, kind) : b.copy(b.p, dev, n, kind);
+    if (e == hipSuccess) e = b.wait();
     if (e == hipSuccess && !toDev) std::memcpy(host, b.p, n);
     return e;
   }
@@ -128,7 +179,7 @@ inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStr
   hipError_t err[kWorkers];
   std::fill(err, err + workers, hipErrorInvalidDevice);  // a worker that never began
   on_workers(workers, device, [&](int w) {
-    StageBlock b[2];
+    StageBlock b[2] = {StageBlock(stream), StageBlock(stream)};
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
     auto ok = [&](hipError_t x) { return (e = x) == hipSuccess; };
@@ -148,12 +199,12 @@ inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStr
         const int s = k & 1;
         if (k >= 2 && !ok(hipEventSynchronize(ev[s]))) break;
         std::memcpy(b[s].p, h + at(i), len(i));
-        if (!ok(hipMemcpyAsync(d + at(i), b[s].p, len(i), kind, stream))) break;
+        if (!ok(b[s].copy(d + at(i), b[s].p, len(i), kind))) break;
         if (!ok(hipEventRecord(ev[s], stream))) break;
       }
     } else {
       auto fetch = [&](size_t j, int s) {
-        return ok(hipMemcpyAsync(b[s].p, d + at(j), len(j), kind, stream)) &&
+        return ok(b[s].copy(b[s].p, d + at(j), len(j), kind)) &&
                ok(hipEventRecord(ev[s], stream));
       };
       if (fetch(i, 0))
@@ -164,9 +215,8 @@ inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStr
           std::memcpy(h + at(i), b[s].p, len(i));
         }
     }
-    // the blocks go back only when nothing on the stream uses them
-    const hipError_t f = hipStreamSynchronize(stream);
-    err[w] = e != hipSuccess ? e : f;
+    const hipError_t f = b[0].wait(), g = b[1].wait();
+    err[w] = e != hipSuccess ? e : f != hipSuccess ? f : g;
     for (auto x : ev)
       if (x) (void)hipEventDestroy(x);
   });
