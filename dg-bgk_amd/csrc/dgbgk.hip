@@ -2371,15 +2371,20 @@ int refresh(Ctx& c, bool sums) {
   return launch_final(c, -1);
 }
 
-// f to or from the reference layout, through the f buffer that holds the
-// previous step (every element of it is rewritten by the next step before it
-// is read): as many input elements a pass as it holds as doubles.
+// f to or from the reference layout, through the larger of two buffers that
+// hold nothing between calls: the f buffer of the previous step (every element
+// of it is rewritten by the next step before it is read) and the update's and
+// seed's moment sums (read by the launch that follows them).  As many input
+// elements a pass as it holds as doubles; in FP32 the f buffer takes half, and
+// small meshes' sums take all (a second pass costs 15 us).
 template <typename T>
 int transfer_f(Ctx& c, double* host, bool toDev) {
   const int E = c.p.E, V = c.p.V;
   const size_t N3 = 3 * (size_t)E;
-  const int per = (int)std::min<size_t>(E, c.ldf * sizeof(T) / (3 * sizeof(double)));
-  double* d = (double*)c.f[1 - c.cur];
+  const size_t fb = (size_t)V * c.ldf * sizeof(T);
+  const size_t mb = (size_t)c.nvchunks * 3 * N3 * sizeof(double);
+  const int per = (int)std::min<size_t>(E, std::max(fb, mb) / (3 * sizeof(double) * V));
+  double* d = mb > fb ? c.msum : (double*)c.f[1 - c.cur];
   T* f = (T*)c.f[c.cur];
   const dim3 g((unsigned)((N3 + 255) / 256), V);
   for (int lo = 0; lo < E; lo += per) {
@@ -2387,7 +2392,7 @@ int transfer_f(Ctx& c, double* host, bool toDev) {
     const size_t bytes = 3 * (size_t)(hi - lo) * V * sizeof(double);
     double* part = host + 3 * (size_t)lo * V;
     if (toDev) {
-      HIPCK(stage_copy(d, part, bytes, true, c.stream, c.dev));
+      HIPCK(stage_copy(d, part, bytes, true, c.stream, c.dev, N3 * V * sizeof(double)));
       hipLaunchKernelGGL(k_to_device<T>, g, dim3(256), 0, c.stream, d, f,
                          (const int*)c.d_eorder, lo, hi, E, V, (long long)c.ldf);
       HIPCK(hipGetLastError());
@@ -2597,10 +2602,13 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   }
   if (const char* fd = std::getenv("DGBGK_FP32_DITHER")) c.dither = fd[0] != '0';
   const Prep& p = c.p;
+  // before the first transfer, whose block the first step then finds
+  StagePool::get().user(1);
   // error path of create: release what was made, report the first error
   auto cleanup = [&](int code) {
     for (void* q : c.owned) (void)hipFree(q);
     if (c.stream) (void)hipStreamDestroy(c.stream);
+    StagePool::get().user(-1);
     delete h;
     return code;
   };
@@ -2721,7 +2729,6 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   if ((st = do_refresh(c, true))) return cleanup(st);
   if (hipStreamSynchronize(c.stream) != hipSuccess)
     return cleanup(fail(kErrHip, "initialisation failed on the device"));
-  StagePool::get().user(1);
   *out = h;
   return kOk;
 }

@@ -25,9 +25,16 @@
 namespace dgbgk {
 
 constexpr size_t kStageBlock = (size_t)2 << 20;
-// f of 26,124 triangles x 256 to the device and back (321 MB): 9.4 ms with
-// one thread, 6.4 with two, 5.3 with three, 4.9 with four (11.7 pageable).
+// f of 26,237 triangles x 128 to the device, a step, and back into a fresh
+// array (81 MB each way): 9.4 ms with one thread, 6.4 with two, 5.3 with
+// three, 4.9 with four (11.7 pageable).
 constexpr int kWorkers = 4;
+// To the device, from arrays up to this size, the runtime's own pageable copy
+// (27 GB/s at 3 MB, 38 at 32 MB): the workers' threads and blocks cost more
+// than they gain.  set_f, ms, with them -> without: 3.2 MB 0.18 -> 0.15, 8 MB
+// 0.36 -> 0.29, 27 MB 0.86 -> 0.82, but 52 MB (past the host's cache) 1.55 ->
+// 1.98.
+constexpr size_t kPageableIn = (size_t)32 << 20;
 
 class StagePool {
  public:
@@ -81,7 +88,8 @@ class StagePool {
 class StageBlock {
  public:
   char* const p;
-  explicit StageBlock(hipStream_t s) : p(StagePool::get().take()), s_(s) {}
+  explicit StageBlock(hipStream_t s, bool wanted = true)
+      : p(wanted ? StagePool::get().take() : nullptr), s_(s) {}
   ~StageBlock() {
     if (!busy_ || hipStreamSynchronize(s_) == hipSuccess) StagePool::get().give(p);
   }
@@ -154,9 +162,10 @@ inline hipError_t stage_fetch(const StagePart* part, int parts, hipStream_t stre
 
 // Copies n bytes between the caller's array and device memory, in order
 // after the work on the stream, and returns when the data has arrived.
-// toDev: host is read, else written.
+// toDev: host is read, else written.  whole: the size of the array this is a
+// part of, if larger.
 inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStream_t stream,
-                             int device) {
+                             int device, size_t whole = 0) {
   const hipMemcpyKind kind = toDev ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
   auto plain = [&](char* d, char* h, size_t m) {
     hipError_t e = toDev ? hipMemcpyAsync(d, h, m, kind, stream) : hipMemcpyAsync(h, d, m, kind, stream);
@@ -173,19 +182,21 @@ inline hipError_t stage_copy(void* dev, void* host, size_t n, bool toDev, hipStr
     if (e == hipSuccess && !toDev) std::memcpy(host, b.p, n);
     return e;
   }
+  if (toDev && std::max(n, whole) <= kPageableIn) return plain((char*)dev, (char*)host, n);
   // each worker takes pieces w, w + workers, ... through two blocks: one on
   // the bus while the other is filled or emptied
   const int workers = (int)std::min<size_t>(kWorkers, pieces);
   hipError_t err[kWorkers];
   std::fill(err, err + workers, hipErrorInvalidDevice);  // a worker that never began
   on_workers(workers, device, [&](int w) {
-    StageBlock b[2] = {StageBlock(stream), StageBlock(stream)};
+    const bool both = (size_t)(w + workers) < pieces;
+    StageBlock b[2] = {StageBlock(stream), StageBlock(stream, both)};
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
     auto ok = [&](hipError_t x) { return (e = x) == hipSuccess; };
     auto at = [&](size_t i) { return i * kStageBlock; };
     auto len = [&](size_t i) { return std::min(kStageBlock, n - at(i)); };
-    const bool staged = b[0].p && (workers == (int)pieces || b[1].p) &&
+    const bool staged = b[0].p && (!both || b[1].p) &&
                         hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) == hipSuccess &&
                         hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) == hipSuccess;
     char *d = (char*)dev, *h = (char*)host;

@@ -46,7 +46,7 @@ static void copies(size_t n, bool toDev) {
   const auto want = bytes(n, (unsigned)n);
   for (long fail_alloc : {-1L, -2L, 1L}) {
     long made = 0;
-    for (long fail = -1; fail <= made; fail += fail < 1 || fail + 2 >= made ? 1 : 3) {
+    for (long fail = -1; fail <= made; fail += fail < 1 || fail + 2 >= made ? 1 : (made + 2) / 3) {
       std::vector<char> host = toDev ? want : std::vector<char>(n), dev(want);
       if (toDev) std::fill(dev.begin(), dev.end(), 0);
       reset(fail, fail_alloc);
@@ -90,11 +90,28 @@ static void fetches() {
     }
 }
 
+// what a short-lived program pays for: a block is made once, and no more of
+// them than pieces or than a transfer needs
+static void few_blocks() {
+  StagePool::get().user(-1);  // empties the pool
+  StagePool::get().user(1);
+  std::vector<char> a(3 * kStageBlock), b(a.size());
+  reset(-1, -1);
+  for (int i = 0; i < 3; ++i) CHECK(stage_copy(b.data(), a.data(), 100, true, &stream, 0) == hipSuccess);
+  CHECK(stub::allocs == 1);
+  CHECK(stage_copy(b.data(), a.data(), a.size(), true, &stream, 0) == hipSuccess);
+  CHECK(stub::allocs == 1);
+  CHECK(stage_copy(b.data(), a.data(), a.size(), false, &stream, 0) == hipSuccess);
+  CHECK(stub::allocs <= 3);
+}
+
 int main() {
   StagePool::get().user(1);
   for (size_t n : {(size_t)1, kStageBlock - 1, kStageBlock, kStageBlock + 1, 3 * kStageBlock,
                    9 * kStageBlock + 5})
     for (bool toDev : {true, false}) copies(n, toDev);
+  copies(kPageableIn + 5, true);
+  few_blocks();
   fetches();
   StagePool::get().user(-1);
   CHECK(stub::live == 0);  // all given back with the last user
