@@ -470,10 +470,10 @@ struct dgbgk_mlp {
   float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // master, Adam, gradient
   bf16* pb = nullptr;                                             // BF16 parameters
   // fused kernels (width <= kMaxFused): hidden weights as operands, the
-  // kernels' activations, pre-activations and dZ, partial sums
+  // pre-activations (then dZ) and activations, partial sums
   bool fused = false;
   bf16 *wf = nullptr, *wb = nullptr;
-  uintx4 *nZ = nullptr, *nA = nullptr, *nD = nullptr;
+  uintx4 *nZ = nullptr, *nA = nullptr;
   float *pw = nullptr, *pin = nullptr, *pout = nullptr, *pbias = nullptr;
   std::vector<bf16*> Z, A;         // per hidden layer, [batch][width]
   bf16 *dZa = nullptr, *dZb = nullptr;
@@ -547,7 +547,7 @@ NetArgs net_args(dgbgk_mlp* h, int rows) {
   a.fin = h->fin; a.fout = h->fout; a.hidden = h->hidden;
   a.pb = h->pb; a.p = h->p; a.wf = h->wf; a.wb = h->wb;
   a.Y = h->Yout; a.loss_part = h->loss_part;
-  a.Z = h->nZ; a.A = h->nA; a.D = h->nD;
+  a.Z = h->nZ; a.A = h->nA;
   a.act4 = (size_t)h->batch * h->width / 8;
   a.pin = h->pin; a.pout = h->pout; a.pbias = h->pbias;
   return a;
@@ -560,11 +560,12 @@ int net_loss_grad(dgbgk_mlp* h, const NetArgs& a) {
   if (st) return st;
   const int W = h->width, L1 = h->hidden - 1, sp = wsplits(a.rows), rper = a.rows / sp;
   const dim3 g(sp, L1), b(256);
+  const uintx4* dz = h->nZ + a.act4;  // of layers 1 .. hidden - 1
   switch (W) {
-    case 64: hipLaunchKernelGGL(k_wgrad<64>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
-    case 128: hipLaunchKernelGGL(k_wgrad<128>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
-    case 192: hipLaunchKernelGGL(k_wgrad<192>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
-    default: hipLaunchKernelGGL(k_wgrad<256>, g, b, 0, h->stream, h->nD, h->nA, a.act4, rper, h->pw); break;
+    case 64: hipLaunchKernelGGL(k_wgrad<64>, g, b, 0, h->stream, dz, h->nA, a.act4, rper, h->pw); break;
+    case 128: hipLaunchKernelGGL(k_wgrad<128>, g, b, 0, h->stream, dz, h->nA, a.act4, rper, h->pw); break;
+    case 192: hipLaunchKernelGGL(k_wgrad<192>, g, b, 0, h->stream, dz, h->nA, a.act4, rper, h->pw); break;
+    default: hipLaunchKernelGGL(k_wgrad<256>, g, b, 0, h->stream, dz, h->nA, a.act4, rper, h->pw); break;
   }
   NetReduce r{h->pw, h->pbias, h->pin, h->pout, h->g, W, h->hidden, h->fin, h->fout, sp,
               net_blocks(a.rows)};
@@ -720,7 +721,6 @@ int dgbgk_mlp_create(int fin, int width, int hidden, int fout, int batch, dgbgk_
     st |= dalloc(h, &h->wb, L1 * ww);
     st |= dalloc(h, &h->nZ, hidden * act4);
     st |= dalloc(h, &h->nA, L1 * act4);
-    st |= dalloc(h, &h->nD, L1 * act4);
     st |= dalloc(h, &h->pw, L1 * sp * ww);
     st |= dalloc(h, &h->pin, nblk * width * (fin + 1));
     st |= dalloc(h, &h->pout, nblk * fout * (width + 1));

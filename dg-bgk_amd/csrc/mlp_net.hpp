@@ -48,10 +48,10 @@ struct NetArgs {
   const bf16* wb;     // and as backward operands
   float* Y;           // [rows][fout] (inference)
   float* loss_part;   // per block
-  uintx4* Z;          // [hidden][rows W/8]: this kernel's own order
+  uintx4* Z;          // [hidden][rows W/8]: this kernel's own order, piece by
+                      // piece where dZ's go
   uintx4* A;          // [hidden-1][rows W/8]: weight-gradient operands
-  uintx4* D;          // dZ of layers 1..hidden-1, the same
-  size_t act4;        // uintx4 per layer of Z, A, D
+  size_t act4;        // uintx4 per layer of Z, A
   float* pin;         // per block: [W][fin+1]  dW, db of the input layer
   float* pout;        //            [fout][W+1] of the output layer
   float* pbias;       // [hidden-1][blocks][W]  db of layers 1..hidden-1
@@ -192,6 +192,8 @@ k_net(NetArgs a) {
     d = mfma(k0, id0, d);
     return mfma(k1, id1, d);
   };
+  // this lane's place in a layer: rows 0-15 of piece nt (16-31: 64 NT on)
+  auto piece = [&](int nt) { return ((size_t)(2 * wave) * NT + nt) * 64 + lane; };
   // a turned piece as the weight-gradient operands of rows 0-15 and 16-31
   auto put = [&](const floatx16& d, uintx4* dst, int nt) {
     unsigned q[8];
@@ -200,8 +202,8 @@ k_net(NetArgs a) {
     uintx4 r0, r1;
     to_operands(q, r0, r1);
     if (live) {
-      dst[((size_t)(2 * wave) * NT + nt) * 64 + lane] = r0;
-      dst[((size_t)(2 * wave + 1) * NT + nt) * 64 + lane] = r1;
+      dst[piece(nt)] = r0;
+      dst[piece(nt) + 64 * NT] = r1;
     }
   };
 
@@ -213,9 +215,9 @@ k_net(NetArgs a) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) p[j] = pk_bf16(z[2 * j], z[2 * j + 1]);
       if (live) {
-        uintx4* zd = a.Z + (size_t)l * a.act4 + ((size_t)wave * NT + nt) * 128 + lane;
+        uintx4* zd = a.Z + (size_t)l * a.act4 + piece(nt);
         zd[0] = uintx4{p[0], p[1], p[2], p[3]};
-        zd[64] = uintx4{p[4], p[5], p[6], p[7]};
+        zd[64 * NT] = uintx4{p[4], p[5], p[6], p[7]};
       }
     }
 #pragma unroll
@@ -354,15 +356,17 @@ k_net(NetArgs a) {
       return s;
     };
     // output layer's gradients and dZ of the last hidden layer
-    uintx4* dl = a.D + (size_t)(H - 2) * a.act4;
+    // (dZ of a layer takes the place of its Z, each lane's values read before
+    // it writes there)
+    uintx4* dl = a.Z + (size_t)(H - 1) * a.act4;
     float* po = a.pout + (size_t)blockIdx.x * fout * (W + 1);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const uintx4* zs = a.Z + (size_t)(H - 1) * a.act4 + ((size_t)wave * NT + nt) * 128 + lane;
+      const uintx4* zs = dl + piece(nt);
       uintx4 z0 = {0, 0, 0, 0}, z1 = z0;
       if (live) {
         z0 = zs[0];
-        z1 = zs[64];
+        z1 = zs[64 * NT];
       }
       const floatx16 d = turn(act[2 * nt], act[2 * nt + 1]);
       {
@@ -429,11 +433,11 @@ k_net(NetArgs a) {
         if (more)
           stage_load(nt + 1 < NT ? a.wb + (size_t)(l - 1) * W * W + (size_t)(nt + 1) * 32 * W
                                  : a.wb + (size_t)(l - 2) * W * W);
-        const uintx4* zs = a.Z + (size_t)(l - 1) * a.act4 + ((size_t)wave * NT + nt) * 128 + lane;
+        const uintx4* zs = a.Z + (size_t)(l - 1) * a.act4 + piece(nt);
         uintx4 z0 = {0, 0, 0, 0}, z1 = z0;
         if (live) {
           z0 = zs[0];
-          z1 = zs[64];
+          z1 = zs[64 * NT];
         }
         const uintx4* wl = s_ring[nt & 1];
         floatx16 acc = {};
@@ -455,7 +459,7 @@ k_net(NetArgs a) {
         for (int r = 0; r < 16; ++r) s += e[r];
         leave(nt & 1, kMaxIO, s);
         if (l > 1) {
-          put(e, a.D + (size_t)(l - 2) * a.act4, nt);
+          put(e, a.Z + (size_t)(l - 1) * a.act4, nt);
         } else {
           float v[FI];
 #pragma unroll
