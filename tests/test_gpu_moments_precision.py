@@ -45,3 +45,26 @@ def test_fp32_sums_are_compensated(rorder, torder, split, monkeypatch):
     assert rms(nf["disux"] - u) < 2e-16 * rms(u)
     assert rms(nf["disuy"] - v) < 1e-16
     assert rms(nf["disps"] / p - 1) < 2e-16
+
+
+@pytest.mark.parametrize("elems,rorder,torder", [(1200, 16, 32), (8000, 8, 16), (8000, 16, 32),
+                                                 (12000, 8, 32)])
+def test_fp64_density_is_no_further_off_than_the_other_kernels(elems, rorder, torder):
+    """FP64 sums are plain; the density of the kernel that holds a node's
+    ordinates within k_moments' own error, 1.2-1.45e-16 RMS of the exact sum
+    at these sizes (a wavefront's 32 ordinates in one chain and its shares in
+    another: 1.7-2.0e-16)."""
+    from dgbgk.solver import Solver
+    case = cylinder_small(elems=elems, rorder=rorder, torder=torder)
+    print(f"case FP64 density {elems} {rorder}x{torder}", flush=True)
+    s = Solver(case)
+    s.step(3)
+    f = s.get_f() * (1 + 0.3 * np.random.default_rng(2).random((s.E, s.V, 3)))
+    s.set_f(f)
+    t, rv, pi = s.tables(), case.prm["rv"], 3.1416
+    w = t["vcord"][:, 2] * (pi * rv * rv * 0.25 * (t["vcord"][:, 0] + 1)) * (4.0 / t["sumweight"])
+    n = np.zeros((s.E, 3), np.longdouble)
+    for v in range(s.V):
+        n += f[:, v].astype(np.longdouble) * np.longdouble(w[v])
+    err = s.node_fields()["disnd"] / n - 1
+    assert float(np.sqrt((err * err).mean())) < 1.4e-16
