@@ -297,7 +297,7 @@ __device__ __forceinline__ bool own_upwind(T w, unsigned cls, int k) {
 // an element and ordinate takes 116 vector and 39 scalar instructions in
 // FP32 (154 and 77 before) and 137 vector ones in FP64 (172), without the
 // tie rule's shifts.  FP32 is bound by them: update 325 -> 306 us at 101,753 x
-// 512, 351 -> 326 us at 26,237 x 2048; FP64 by memory: 626 -> 629 us.
+// 512, 351 -> 326 us at 27,817 x 2048; FP64 by memory: 626 -> 629 us.
 template <typename T>
 struct OrdRow {
   T ux, uy, fin, ph;   // velocity, inflow value, FP32 store dither phase
@@ -2585,7 +2585,7 @@ int dgbgk_create(int nelem, int npoin, int nboun, const int* intma, const double
   // ordinates of f in flight per update thread beyond the one computed, and
   // whether the update kernel also sums the first moment pass.  FP32: two (96
   // registers, as many wavefronts per SIMD as with one: update 306 -> 298 us
-  // at 101,753 x 512, 326 -> 314 us at 25,781 x 2048, 11.60 -> 11.36 ms at
+  // at 101,753 x 512, 326 -> 314 us at 27,817 x 2048, 11.60 -> 11.36 ms at
   // 1,005,669 x 2048) where the chip's 256 x 5 resident blocks walk 16
   // ordinates each or more; shorter chunks gain nothing from it (21.1 against
   // 21.3 us at 5,763 x 128).  FP64: one (629 -> 636 us with two).
